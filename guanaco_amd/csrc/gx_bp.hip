@@ -20,8 +20,11 @@
 // kBF16 (whose error budget is set by the storage) compute p with two fused
 // multiply-adds from a table holding offset - 1/2 and the scale times the
 // normalisation the filter pass divided out, and accumulate with FP32 fused
-// multiply-adds (BF16 taps rounded to FP16 first: bf16_tap). The per-tilt
-// tables are read with scalar loads.
+// multiply-adds (BF16 taps rounded to FP16 first: bf16_tap); here they have
+// the direct kernels only (narrow slabs, one centre per row), the other
+// plans run on the matrix cores (gx_bp_mm.hip). The per-tilt tables are read
+// with scalar loads.
+#include "gx_bp_geometry.hpp"
 #include "gx_common.hpp"
 #include "gx_kernels.hpp"
 
@@ -29,42 +32,16 @@ namespace gx {
 
 constexpr int kTX = 32, kTZ = 8;
 
-// Per-tilt tables are read through the constant address space: uniform
-// indices become scalar loads, independent of the workgroup barriers.
-typedef const __attribute__((address_space(4))) float kfloat;
-typedef const __attribute__((address_space(4))) int kint;
-
-__device__ __forceinline__ float4 kload(const float4 *p, size_t i) {
-  kfloat *q = (kfloat *)p + 4 * i;
-  return make_float4(q[0], q[1], q[2], q[3]);
-}
-__device__ __forceinline__ int2 kload(const int2 *p, size_t i) {
-  kint *q = (kint *)p + 2 * i;
-  return make_int2(q[0], q[1]);
-}
-__device__ __forceinline__ float kload(const float *p, size_t i) {
-  return ((kfloat *)p)[i];
-}
-
 template <int YB, int STORE>
 struct Taps;
 
-// BF16 taps enter the arithmetic rounded to FP16, as the staged kernel keeps
-// them in LDS (bf16_pair_to_f16): exact for magnitudes in [2^-14, 65504]
-// (eight significant bits fit FP16's eleven), and within 2^-25 below, where
-// FP16 is subnormal. The normalised slabs stay far below 65504, as they must
-// for FP16 storage. The staged kernel then interpolates with
-// v_fma_mix_f32, one instruction per tap, like FP16, where BF16 would need a
-// shift or mask before each FMA; the direct kernels round the same way so
-// that every kernel gives the same bits.
+// BF16 taps enter the arithmetic rounded to FP16, as the matrix-core kernel
+// keeps them in LDS: exact for magnitudes in [2^-14, 65504] (eight
+// significant bits fit FP16's eleven), and within 2^-25 below, where FP16 is
+// subnormal. The normalised slabs stay far below 65504, as they must for FP16
+// storage.
 __device__ __forceinline__ float bf16_tap(float v) {
   return (float)(_Float16)v;
-}
-__device__ __forceinline__ uint32_t bf16_pair_to_f16(uint32_t w) {
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-  const f32x2 f = {__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u)};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
 }
 template <int STORE>
 __device__ __forceinline__ float tap_value(typename StoreT<STORE>::T v) {
@@ -137,13 +114,6 @@ struct Taps {
 #pragma unroll
     for (int i = 0; i < YB / 8; ++i) unpack(i, q0[i], q1[i]);
   }
-  // The staged kernel's word-major runs: word i of position p at q[i SW]
-  // (q at position p), position p + 1 one word on.
-  template <int SW>
-  __device__ __forceinline__ void load16_strided(const uint4 *q) {
-#pragma unroll
-    for (int i = 0; i < YB / 8; ++i) unpack(i, q[i * SW], q[i * SW + 1]);
-  }
   __device__ __forceinline__ static float lo(uint32_t w) {
     if constexpr (STORE == kF16) {
       return __half2float(__ushort_as_half((unsigned short)(w & 0xffffu)));
@@ -160,78 +130,52 @@ struct Taps {
   }
 };
 
-// reconstructor.cpp:56-58: half-integer voxel centres (exact in float).
-__device__ __forceinline__ float voxel_coord(int i, int n) {
-  return (float)((double)i - 0.5 * (double)n + 0.5);
-}
-
-// reconstructor.cpp:59-60,76-79: detector position p = x c - z s + offset,
-// i0 = floor(p - 0.5), t = (p - 0.5) - i0. EXACT: the reference's operation
-// order; otherwise cf.z already holds offset - 1/2 and p is two fused
-// multiply-adds.
-template <bool EXACT>
-__device__ __forceinline__ int tap_index(float x, float z, float4 cf,
-                                         float &tt) {
-  float p;
-  if constexpr (EXACT) {
-    p = x * cf.x - z * cf.y + cf.z;
-    p = p - 0.5f;
-  } else {
-    p = fmaf(x, cf.x, fmaf(-z, cf.y, cf.z));
-  }
-  const float fi = floorf(p);
-  tt = p - fi;
-  return (int)fi;
-}
-
-// reconstructor.cpp:66-73: slab k = clamp(floor(h * dscale + doffset + 0.5)),
-// h = -x s - z c. floor((double)d + 0.5) without FP64: round half to even,
-// then move exact ties up.
-__device__ __forceinline__ float slab_coord(float x, float z, float4 cf,
-                                            float dscale, float doffset) {
-  const float h = -x * cf.y - z * cf.x;
-  return h * dscale + doffset;
-}
-__device__ __forceinline__ int slab_of(float x, float z, float4 cf,
-                                       float dscale, float doffset, int ndf) {
-  const float d = slab_coord(x, z, cf, dscale, doffset);
-  float n = rintf(d);
-  if (d - n == 0.5f) n += 1.0f;
-  return min(max((int)n, 0), ndf - 1);
-}
-
 // ------------------------------------------------------- per-tilt tables --
 
 // out[t] = (c, s, offset - 1/2, scale * normalisation): the normalisation
 // float(tmax[t]) * nrm_mul is what the filter pass divided the stored values
-// by (1 where it is not positive, or without tmax). Entries past T are zero.
-__global__ void k_bp_coefficients(const float4 *__restrict__ coef,
-                                  const uint32_t *__restrict__ tmax,
-                                  float nrm_mul, int T, int Tpad,
-                                  float4 *__restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= Tpad) return;
-  float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (t < T) {
-    const float4 cf = coef[t];
-    float nrm = tmax != nullptr ? __uint_as_float(tmax[t]) * nrm_mul : 1.0f;
-    if (!(nrm > 0.0f)) nrm = 1.0f;
-    r = make_float4(cf.x, cf.y, cf.z - 0.5f, cf.w * nrm);
+// by (1 where it is not positive, or without tmax). Entries T .. Tpad - 1 are
+// zero; entry Tpad holds (u, 1 / u): the power of two u that takes the
+// largest finite |scale| to [2^13, 2^14) (1 where there is none). One
+// workgroup.
+__global__ __launch_bounds__(256) void k_bp_coefficients(
+    const float4 *__restrict__ coef, const uint32_t *__restrict__ tmax,
+    float nrm_mul, int T, int Tpad, float4 *__restrict__ out) {
+  __shared__ float red[4];
+  float top = 0.0f;
+  for (int t = threadIdx.x; t < Tpad; t += 256) {
+    float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (t < T) {
+      const float4 cf = coef[t];
+      float nrm = tmax != nullptr ? __uint_as_float(tmax[t]) * nrm_mul : 1.0f;
+      if (!(nrm > 0.0f)) nrm = 1.0f;
+      r = make_float4(cf.x, cf.y, cf.z - 0.5f, cf.w * nrm);
+      const float a = fabsf(r.w);
+      if (a < __builtin_inff()) top = fmaxf(top, a);
+    }
+    out[t] = r;
   }
-  out[t] = r;
+  top = block_max<256>(top, red);
+  if (threadIdx.x == 0) {
+    int e = 0;
+    if (top > 0.0f) {
+      (void)frexpf(top, &e);  // top in [2^(e-1), 2^e)
+      e = min(max(14 - e, -126), 126);
+    }
+    out[Tpad] = make_float4(ldexpf(1.0f, e), ldexpf(1.0f, -e), 0.0f, 0.0f);
+  }
 }
 
 hipError_t launch_bp_coefficients(const float4 *coef, const uint32_t *tmax,
                                   float nrm_mul, int T, float4 *out,
                                   hipStream_t s) {
-  const int Tpad = bp_tilt_pad(T);
-  hipLaunchKernelGGL(k_bp_coefficients, dim3((Tpad + 63) / 64), dim3(64), 0, s,
-                     coef, tmax, nrm_mul, T, Tpad, out);
+  hipLaunchKernelGGL(k_bp_coefficients, dim3(1), dim3(256), 0, s, coef, tmax,
+                     nrm_mul, T, bp_tilt_pad(T), out);
   return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
-// LDS-staged form.
+// LDS-staged form (float32 slabs).
 //
 // p is a chain of correctly rounded float operations, each monotone in x and
 // in z, so over a 32 x 8 tile i0 is smallest at one of the four corners, and
@@ -251,15 +195,13 @@ hipError_t launch_bp_coefficients(const float4 *coef, const uint32_t *tmax,
 // values, never an access outside the buffer.
 //
 // The runs are loaded straight into LDS (buffer_load ... lds), not through
-// registers; BF16 runs are then converted to FP16 in place by the lanes that
-// loaded them (bf16_tap). Two LDS buffers: the loads of batch b + 1 are
-// issued before batch b is interpolated, one barrier per batch.
+// registers. Two LDS buffers: the loads of batch b + 1 are issued before
+// batch b is interpolated, one barrier per batch. FP32 slabs only.
 constexpr int kWPOS = 40;
 
-template <int YB, int STORE, int KS>
+template <int YB, int KS>
 struct Staging {
-  using T = typename StoreT<STORE>::T;
-  static constexpr int kPosBytes = YB * (int)sizeof(T);
+  static constexpr int kPosBytes = YB * (int)sizeof(float);
   static constexpr int kPosWords = kPosBytes / 16;      // 16-byte words
   static constexpr int kTB = 256 / (kPosBytes * KS);    // tilts per batch
   static constexpr int kNSlot = kTB * KS;  // (tilt, slab) runs per batch
@@ -279,14 +221,6 @@ struct Staging {
   static_assert(kNSlot % (kTX * kTZ / 64) == 0, "runs split evenly on waves");
 };
 
-// One 16-byte raw buffer load per lane, written to LDS at dst + 16 lane
-// instead of to registers (M0 holds dst). Out-of-range offsets write zeros.
-__device__ __forceinline__ void load_to_lds16(__amdgpu_buffer_rsrc_t rs,
-                                              uint4 *dst, int off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(
-      rs, (__attribute__((address_space(3))) void *)dst, 16, off, 0, 0, 0);
-}
-
 // Window of one tilt over the tile's active voxels [x0, x1] x [z0, z1]:
 // smallest i0 and smallest k over the four corners, with kOneSlab set in .y
 // when the largest k over the corners is the same: slab_of is monotone in x
@@ -294,7 +228,7 @@ __device__ __forceinline__ void load_to_lds16(__amdgpu_buffer_rsrc_t rs,
 constexpr int kOneSlab = 1 << 30;
 constexpr int kSlabMask = kOneSlab - 1;
 
-template <bool EXACT, bool MULTI>
+template <bool MULTI>
 __device__ __forceinline__ int2 tile_window(float4 cf, float x0, float x1,
                                             float z0, float z1, float dscale,
                                             float doffset, int ndf) {
@@ -304,7 +238,7 @@ __device__ __forceinline__ int2 tile_window(float4 cf, float x0, float x1,
     const float x = (c & 1) ? x1 : x0;
     const float z = (c & 2) ? z1 : z0;
     float tt;
-    w = min(w, tap_index<EXACT>(x, z, cf, tt));
+    w = min(w, tap_index<true>(x, z, cf, tt));
     if constexpr (MULTI) {
       const int kc = slab_of(x, z, cf, dscale, doffset, ndf);
       k = min(k, kc);
@@ -315,7 +249,7 @@ __device__ __forceinline__ int2 tile_window(float4 cf, float x0, float x1,
 }
 
 // win[tile * Tpad + t], tile = bx * nbz + bz (the kernels' order).
-template <bool EXACT, bool MULTI>
+template <bool MULTI>
 __global__ void k_bp_windows(const float4 *__restrict__ coef, int T, int Tpad,
                              int W, int Z, int nbx, int nbz, float dscale,
                              float doffset, int ndf, int2 *__restrict__ win) {
@@ -330,8 +264,7 @@ __global__ void k_bp_windows(const float4 *__restrict__ coef, int T, int Tpad,
     const float x1 = voxel_coord(min(bx * kTX + kTX, W) - 1, W);
     const float z0 = voxel_coord(bz * kTZ, Z);
     const float z1 = voxel_coord(min(bz * kTZ + kTZ, Z) - 1, Z);
-    r = tile_window<EXACT, MULTI>(coef[t], x0, x1, z0, z1, dscale, doffset,
-                                  ndf);
+    r = tile_window<MULTI>(coef[t], x0, x1, z0, z1, dscale, doffset, ndf);
   }
   win[i] = r;
 }
@@ -341,26 +274,19 @@ size_t bp_window_entries(int W, int Z, int T) {
   return nbx * nbz * (size_t)bp_tilt_pad(T);
 }
 
-hipError_t launch_bp_windows(const float4 *coef, int exact, int T, int W,
-                             int Z, float dscale, float doffset, int ndf,
-                             int2 *win, hipStream_t s) {
+hipError_t launch_bp_windows(const float4 *coef, int T, int W, int Z,
+                             float dscale, float doffset, int ndf, int2 *win,
+                             hipStream_t s) {
   const int nbx = (W + kTX - 1) / kTX, nbz = (Z + kTZ - 1) / kTZ;
   const size_t n = bp_window_entries(W, Z, T);
   const dim3 g((unsigned)((n + 255) / 256)), b(256);
   const int Tpad = bp_tilt_pad(T);
-  const bool multi = ndf > 1;
-  if (exact && multi)
-    hipLaunchKernelGGL((k_bp_windows<true, true>), g, b, 0, s, coef, T, Tpad,
-                       W, Z, nbx, nbz, dscale, doffset, ndf, win);
-  else if (exact)
-    hipLaunchKernelGGL((k_bp_windows<true, false>), g, b, 0, s, coef, T, Tpad,
-                       W, Z, nbx, nbz, dscale, doffset, ndf, win);
-  else if (multi)
-    hipLaunchKernelGGL((k_bp_windows<false, true>), g, b, 0, s, coef, T, Tpad,
-                       W, Z, nbx, nbz, dscale, doffset, ndf, win);
+  if (ndf > 1)
+    hipLaunchKernelGGL(k_bp_windows<true>, g, b, 0, s, coef, T, Tpad, W, Z,
+                       nbx, nbz, dscale, doffset, ndf, win);
   else
-    hipLaunchKernelGGL((k_bp_windows<false, false>), g, b, 0, s, coef, T, Tpad,
-                       W, Z, nbx, nbz, dscale, doffset, ndf, win);
+    hipLaunchKernelGGL(k_bp_windows<false>, g, b, 0, s, coef, T, Tpad, W, Z,
+                       nbx, nbz, dscale, doffset, ndf, win);
   return hipGetLastError();
 }
 
@@ -513,19 +439,16 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_rows(
   }
 }
 
-template <int YB, int STORE, bool MULTI, int KS>
+template <int YB, bool MULTI, int KS>
 __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
-    const typename StoreT<STORE>::T *__restrict__ slab,
+    const float *__restrict__ slab,
     const float4 *__restrict__ coef, const int2 *__restrict__ win,
     float dscale, float doffset, int ndf, int N, int T, int NYB, int W, int Z,
     int Y, int yb0, int y_base, int slab_yb0, float *__restrict__ vol,
     int nbx, int nbz,
     unsigned nblocks) {
-  using S = Staging<YB, STORE, KS>;
-  using ST = typename StoreT<STORE>::T;
-  constexpr bool kExact = STORE == kF32;
-  // BF16 runs are staged as FP16 (bf16_tap)
-  constexpr int kLds = STORE == kBF16 ? kF16 : STORE;
+  using S = Staging<YB, KS>;
+  using ST = float;
   static_assert(MULTI || KS == 1, "one slab without defocus slabs");
   // Two buffers as two arrays: with distinct objects the compiler can tell
   // that reads of one do not wait for the direct loads into the other.
@@ -591,24 +514,6 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
                       dslot[c] >= 0 ? base + dslot[c] : -1);
     }
   };
-  // After this wave's loads have landed: BF16 slots to FP16, each by the
-  // lane that loaded it (no other wave touches them before the barrier).
-  auto convert_batch = [&](uint4 *dst) {
-    if constexpr (STORE == kBF16) {
-#pragma unroll
-      for (int i = 0; i < S::kSPW; ++i) {
-        const int q = wave + (kTX * kTZ / 64) * i;
-#pragma unroll
-        for (int c = 0; c < S::kCPL; ++c) {
-          uint4 *d = dst + q * S::kRunSlots + lane + 64 * c;
-          const uint4 v = *d;
-          *d = make_uint4(bf16_pair_to_f16(v.x), bf16_pair_to_f16(v.y),
-                          bf16_pair_to_f16(v.z), bf16_pair_to_f16(v.w));
-        }
-      }
-    }
-  };
-
   float acc[YB];
 #pragma unroll
   for (int r = 0; r < YB; ++r) acc[r] = 0.0f;
@@ -644,14 +549,14 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
           }
         }
         float tt;
-        const int i0 = tap_index<kExact>(x, z, cf, tt);
+        const int i0 = tap_index<true>(x, z, cf, tt);
         if (active && (unsigned)i0 < (unsigned)(N - 1)) {
           const int rel = min(max(i0 - w.x, 0), kWPOS - 2);
           // word-major run: word wi of position p in slot wi kWPOS + p
-          Taps<YB, kLds> tp;
+          Taps<YB, kF32> tp;
           tp.template load16_strided<kWPOS>(cur + (j * KS + ks) * S::kRunSlots +
                                             rel);
-          accumulate<YB, kLds>(acc, tp, cf, tt);
+          accumulate<YB, kF32>(acc, tp, cf, tt);
         }
       }
     }
@@ -659,14 +564,12 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
       // this wave's loads have landed; the barrier then covers the other
       // waves' too
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      convert_batch(nxt);
     }
     lds_barrier();
   };
 
   load_batch(0, lds_a);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  convert_batch(lds_a);
   lds_barrier();
   const int nb = (T + S::kTB - 1) / S::kTB;
   for (int b = 0; b < nb; b += 2) {
@@ -683,28 +586,27 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
 }
 
 // ------------------------------------------------------------ launchers ---
-template <int YB, int STORE, bool MULTI, int KS>
+template <int YB, bool MULTI, int KS>
 static hipError_t launch_bp_lds_k(const BpArgs &a, hipStream_t s) {
-  using ST = typename StoreT<STORE>::T;
   const int nbx = (a.W + kTX - 1) / kTX;
   const int nbz = (a.Z + kTZ - 1) / kTZ;
   if (a.yb1 <= a.yb0) return hipSuccess;
   if (a.win == nullptr) return hipErrorInvalidValue;
   const unsigned nb =
       (unsigned)nbx * (unsigned)nbz * (unsigned)(a.yb1 - a.yb0);
-  hipLaunchKernelGGL((k_bp_lds<YB, STORE, MULTI, KS>), dim3(nb),
-                     dim3(kTX * kTZ), 0, s, (const ST *)a.slab, a.coef, a.win,
-                     a.dscale, a.doffset, a.ndf, a.N, a.T, a.NYB, a.W, a.Z,
-                     a.Y, a.yb0, a.y_base, a.slab_yb0, a.vol, nbx, nbz, nb);
+  hipLaunchKernelGGL((k_bp_lds<YB, MULTI, KS>), dim3(nb), dim3(kTX * kTZ), 0,
+                     s, (const float *)a.slab, a.coef, a.win, a.dscale,
+                     a.doffset, a.ndf, a.N, a.T, a.NYB, a.W, a.Z, a.Y, a.yb0,
+                     a.y_base, a.slab_yb0, a.vol, nbx, nbz, nb);
   return hipGetLastError();
 }
 
-template <int YB, int STORE>
+template <int YB>
 static hipError_t launch_bp_lds_t(const BpArgs &a, hipStream_t s) {
-  if (a.ndf == 1) return launch_bp_lds_k<YB, STORE, false, 1>(a, s);
+  if (a.ndf == 1) return launch_bp_lds_k<YB, false, 1>(a, s);
   switch (a.staged) {
-    case 2: return launch_bp_lds_k<YB, STORE, true, 2>(a, s);
-    case 4: return launch_bp_lds_k<YB, STORE, true, 4>(a, s);
+    case 2: return launch_bp_lds_k<YB, true, 2>(a, s);
+    case 4: return launch_bp_lds_k<YB, true, 4>(a, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -756,6 +658,7 @@ static hipError_t launch_bp_rows_t(const BpArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_bp(const BpArgs &a, int YB, int store, hipStream_t s) {
+  if (a.mm) return launch_bp_mm(a, YB, store, s);
   if (a.row_off != nullptr) {
     if (store == kF32) {
       if (YB == 8) return launch_bp_rows_t<8, kF32>(a, s);
@@ -770,16 +673,8 @@ hipError_t launch_bp(const BpArgs &a, int YB, int store, hipStream_t s) {
     return hipErrorInvalidValue;
   }
   if (a.staged) {
-    if (store == kF32) {
-      if (YB == 8) return launch_bp_lds_t<8, kF32>(a, s);
-      if (YB == 16) return launch_bp_lds_t<16, kF32>(a, s);
-    } else if (store == kF16) {
-      if (YB == 16) return launch_bp_lds_t<16, kF16>(a, s);
-      if (YB == 32) return launch_bp_lds_t<32, kF16>(a, s);
-    } else if (store == kBF16) {
-      if (YB == 16) return launch_bp_lds_t<16, kBF16>(a, s);
-      if (YB == 32) return launch_bp_lds_t<32, kBF16>(a, s);
-    }
+    if (store == kF32 && YB == 8) return launch_bp_lds_t<8>(a, s);
+    if (store == kF32 && YB == 16) return launch_bp_lds_t<16>(a, s);
     return hipErrorInvalidValue;
   }
   if (store == kF32) {

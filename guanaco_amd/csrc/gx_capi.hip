@@ -774,6 +774,9 @@ struct gx_volume_plan {
   int band = 0, slab_y0 = 0, slab_y1 = 0;
   int bp_kind = GX_BP_STAGED;
   int bp_staged = 1;  // slabs per tilt of the staged kernel; 0 = direct
+  // 16-bit slabs of a plan with one centre whose tiles span at most
+  // bp_staged slabs: both kinds run the matrix-core kernel
+  bool bp_mm = false;
   bool ctf = false;
   float dscale = 0, doffset = 0, nrm_mul = 1;
   size_t slab_bytes = 0, total_bytes = 0;
@@ -897,6 +900,19 @@ struct PlanSizes {
   size_t slab_bytes, mask_bytes, f_bytes, g_bytes, small_bytes, total;
 };
 
+// Whether a plan backprojects on the matrix cores, and the entries of its
+// window table.
+bool plan_mm(const gx_volume_desc *d) {
+  float dscale, doffset;
+  defocus_coefficients(d->num_defocus, d->pixel_size, d->min_defocus,
+                       d->max_defocus, &dscale, &doffset);
+  return d->storage != GX_STORE_F32 && d->centres == nullptr &&
+         bp_slots(d->num_defocus, dscale) != 0;
+}
+size_t plan_windows(int W, int Z, int T, bool mm) {
+  return mm ? bp_mm_window_entries(W, Z, T) : bp_window_entries(W, Z, T);
+}
+
 int plan_sizes(const gx_volume_desc *d, PlanSizes *ps) {
   GX_CHECK(d != nullptr);
   GX_CHECK(d->num_pixels > 0 && d->num_rows > 0 && d->num_angles > 0);
@@ -968,9 +984,10 @@ int plan_sizes(const gx_volume_desc *d, PlanSizes *ps) {
     ps->f_bytes = ps->g_bytes = 0;
   }
   ps->chunk = (int)chunk;
-  ps->small_bytes = (size_t)bp_tilt_pad((int)T) * 2 * sizeof(float4) +
+  ps->small_bytes = ((size_t)bp_tilt_pad((int)T) * 2 + 1) * sizeof(float4) +
                     T * 2 * sizeof(float) +
-                    bp_window_entries((int)d->width, (int)d->depth, (int)T) *
+                    plan_windows((int)d->width, (int)d->depth, (int)T,
+                                 plan_mm(d)) *
                         sizeof(int2) +
                     sizeof(float) * (ps->L / 2 + 1) + sizeof(double) * ndf +
                     (d->centres ? sizeof(float) * T * Y : 0) +
@@ -1024,6 +1041,7 @@ void plan_setup(gx_volume_plan *p, const gx_volume_desc *d,
   p->per_row = d->centres != nullptr;
   p->bp_staged = p->per_row ? 0 : bp_slots(d->num_defocus, p->dscale);
   p->bp_kind = p->bp_staged ? GX_BP_STAGED : GX_BP_DIRECT;
+  p->bp_mm = plan_mm(d);
   apply_tuned(p);
   const size_t T = d->num_angles;
   if (p->per_row) {
@@ -1081,8 +1099,9 @@ void plan_buffers(gx_volume_plan *p, const PlanSizes &ps,
   const size_t T = p->T, Tpad = (size_t)bp_tilt_pad(p->T);
   out = {{&p->slab, ps.slab_bytes},
          {&p->coef, sizeof(float4) * Tpad},
-         {&p->coef_r, sizeof(float4) * Tpad},
-         {&p->win, sizeof(int2) * bp_window_entries(p->W, p->Z, p->T)},
+         {&p->coef_r, sizeof(float4) * (Tpad + 1)},
+         {&p->win,
+          sizeof(int2) * plan_windows(p->W, p->Z, p->T, p->bp_mm)},
          {&p->wscale, sizeof(float) * T},
          {&p->tmax, sizeof(uint32_t) * T},
          {&p->ramp, sizeof(float) * p->h_ramp.size()},
@@ -1103,15 +1122,16 @@ int plan_upload(gx_volume_plan *p, hipStream_t s) {
                         hipMemcpyHostToDevice, s));
   // the staged kernel's windows, with the arithmetic of the plan's kernels
   if (p->storage == GX_STORE_F32) {
-    GX_HIP(launch_bp_windows(p->coef.as<float4>(), 1, p->T, p->W, p->Z,
+    GX_HIP(launch_bp_windows(p->coef.as<float4>(), p->T, p->W, p->Z,
                              p->dscale, p->doffset, p->ndf, p->win.as<int2>(),
                              s));
   } else {
     GX_HIP(launch_bp_coefficients(p->coef.as<float4>(), nullptr, 1.0f, p->T,
                                   p->coef_r.as<float4>(), s));
-    GX_HIP(launch_bp_windows(p->coef_r.as<float4>(), 0, p->T, p->W, p->Z,
-                             p->dscale, p->doffset, p->ndf, p->win.as<int2>(),
-                             s));
+    if (p->bp_mm)
+      GX_HIP(launch_bp_mm_windows(p->coef_r.as<float4>(), p->T, p->W, p->Z,
+                                  p->dscale, p->doffset, p->ndf,
+                                  p->win.as<int2>(), s));
   }
   // the slabs each tilt's voxels read, and the (tilt, defocus) list
   if (p->ndf > 1) {
@@ -1356,6 +1376,7 @@ extern "C" int gx_volume_backproject_rows(gx_volume_plan *p, size_t y0,
   a.y_base = (int)y0;
   a.slab_yb0 = p->slab_y0 / p->YB;
   a.vol = d_vol;
+  a.mm = p->bp_mm;
   a.staged = p->bp_kind == GX_BP_STAGED ? p->bp_staged : 0;
   a.row_off = p->per_row ? p->row_off.as<float>() : nullptr;
   a.Y_tab = p->Y;
@@ -1492,16 +1513,22 @@ extern "C" int gx_volume_plan_autotune(gx_volume_plan *p, const float *d_in,
     GX_HIP(hipEventSynchronize(ev.b));
     float fms = 0.0f;
     GX_HIP(hipEventElapsedTime(&fms, ev.a, ev.b));
+    float bms = 0.0f;
     for (int kind : kinds) {
       if (!tile_valid(p, rows[ri], kind)) continue;
       p->bp_kind = kind;
+      // (the matrix-core kernel runs for both kinds: timed once)
+      if (p->bp_mm && kind != kinds[0]) {
+        GX_CHECK(r.n < GX_TUNE_MAX);
+        r.cand[r.n++] = gx_tune_entry{kind, rows[ri], fms, bms};
+        continue;
+      }
       if ((rc = gx_volume_backproject_rows(p, 0, yt, d_vol, s))) return rc;
       GX_HIP(hipEventRecord(ev.a, s));
       for (int i = 0; i < 2; ++i)
         if ((rc = gx_volume_backproject_rows(p, 0, yt, d_vol, s))) return rc;
       GX_HIP(hipEventRecord(ev.b, s));
       GX_HIP(hipEventSynchronize(ev.b));
-      float bms = 0.0f;
       GX_HIP(hipEventElapsedTime(&bms, ev.a, ev.b));
       bms *= 0.5f;
       GX_CHECK(r.n < GX_TUNE_MAX);

@@ -37,6 +37,8 @@ struct BpArgs {
   // row y (kF32: the reference's offset; reduced: offset - 1/2), or null
   const float *row_off;
   int Y_tab;
+  bool mm;                   // 16-bit slabs on the matrix cores
+                             // (launch_bp_mm); `staged` is then not read
   int staged;                // 0: direct kernel; 2 or 4 (or 1 with one slab):
                              // LDS-staged kernel holding that many slabs
 };
@@ -139,16 +141,28 @@ hipError_t launch_absmax_rows(const float *src, size_t st, size_t sk,
 // store: kF32 (exact reference arithmetic) or kF16/kBF16 (FP32 accumulate).
 hipError_t launch_bp(const BpArgs &a, int YB, int store, hipStream_t s);
 // Reduced-storage coefficient table from the reference's (c, s, offset,
-// scale) and the per-tilt normalisation of the filter pass.
+// scale) and the per-tilt normalisation of the filter pass:
+// bp_tilt_pad(T) + 1 entries, the last the power of two that scales the
+// weights of launch_bp_mm, and its inverse.
 hipError_t launch_bp_coefficients(const float4 *coef, const uint32_t *tmax,
                                   float nrm_mul, int T, float4 *out,
                                   hipStream_t s);
-// Window table of the staged kernel: bp_window_entries(W, Z, T) int2, from
-// the coefficient table the kernels read (exact != 0: kF32 arithmetic).
+// Window table of the staged kernel (float32 slabs): bp_window_entries(W, Z,
+// T) int2, from the reference's coefficients.
 size_t bp_window_entries(int W, int Z, int T);
-hipError_t launch_bp_windows(const float4 *coef, int exact, int T, int W,
-                             int Z, float dscale, float doffset, int ndf,
+hipError_t launch_bp_windows(const float4 *coef, int T, int W, int Z,
+                             float dscale, float doffset, int ndf,
                              int2 *win, hipStream_t s);
+
+// The matrix-core kernel of 16-bit slabs (one centre, a tile spans at most
+// four slabs; a.win from launch_bp_mm_windows): any rows per block YB that
+// the storage has.
+hipError_t launch_bp_mm(const BpArgs &a, int YB, int store, hipStream_t s);
+// Its window table, bp_mm_window_entries(W, Z, T) int2.
+size_t bp_mm_window_entries(int W, int Z, int T);
+hipError_t launch_bp_mm_windows(const float4 *coef, int T, int W, int Z,
+                                float dscale, float doffset, int ndf,
+                                int2 *win, hipStream_t s);
 
 // Seeded synthetic tilt series (ellipsoid phantom, optional CTF, noise).
 struct SynthArgs {

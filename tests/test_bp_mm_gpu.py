@@ -1,0 +1,128 @@
+"""The matrix-core backprojector of 16-bit slabs at the edges of its tiles.
+
+Each plan's own decoded slabs (times the per-tilt normalisation the filter
+divided out) are backprojected by the FP32 oracle. What is left is the FP32
+rounding of both sides and the weights' split into two FP16 parts: at most
+2^-22 per weight, and about (T + 8) 2^-24 of the sum of the terms'
+magnitudes in the accumulation, below 5e-6 for the 64 tilts used here at
+most; 1e-5 with the oracle's own rounding.
+"""
+import numpy
+import pytest
+
+from guanaco_amd import _capi as C
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# X, Y, T, ndf, Z, W, last tilt (deg), (min_df, max_df), weights
+CASES = [
+    # one voxel, one row, one tilt
+    (8, 1, 1, 1, 1, 1, 0.0, (0.0, 0.0), None),
+    # partial 4 x 4 blocks and tiles, odd width, one 32-row block
+    (70, 31, 3, 1, 17, 67, 60.0, (0.0, 0.0), None),
+    # two row blocks, the second partial; whole batches of four tilts
+    (64, 33, 8, 1, 16, 64, 60.0, (0.0, 0.0), None),
+    # four row blocks, and one row into the next workgroup
+    (48, 129, 5, 1, 33, 50, 80.0, (0.0, 0.0), None),
+    # every quadrant, a detector narrower than a staged run
+    (20, 65, 64, 1, 40, 36, 175.0, (0.0, 0.0), None),
+    # two and three slabs in a tile: extra runs, batches that close early
+    (96, 40, 21, 6, 50, 96, 65.0, (-100.0, 100.0), None),
+    (80, 97, 30, 4, 80, 80, 70.0, (-25.0, 25.0), None),
+    # tilts of very different weight
+    (64, 34, 12, 2, 20, 64, 60.0, (-90.0, 90.0), 1e-3),
+]
+
+
+def plan_of(case, storage):
+    X, Y, T, ndf, Z, W, last, (mn, mx), weights = case
+    angles = numpy.deg2rad(numpy.linspace(-last, last, T)).astype(
+        numpy.float32)
+    rng = numpy.random.default_rng(X + Y + T + ndf)
+    sino = rng.standard_normal((Y, ndf, T, X)).astype(numpy.float32)
+    w = numpy.ones(T, numpy.float32)
+    if weights is not None:
+        w = numpy.geomspace(1.0, weights, T).astype(numpy.float32)
+    plan = C.VolumePlan(X, Y, angles, Z, width=W, num_defocus=ndf,
+                        centre=X / 2.0 - 0.3, min_defocus=mn, max_defocus=mx,
+                        weights=w, storage=storage,
+                        input_layout=C.INPUT_SINOGRAMS)
+    assert plan.backprojector()[1] > 0
+    return plan, sino, angles
+
+
+def run(plan, case, sino):
+    X, Y, T, ndf, Z, W = case[:6]
+    d_in = C.DeviceArray.from_host(sino)
+    d_vol = C.DeviceArray((Y, Z, W))
+    C.call("gx_fill_u32", d_vol.ptr, 0x7fc00000, Y * Z * W, None)
+    plan.run(d_in, d_vol)
+    C.call("gx_device_synchronize")
+    return d_vol.to_host()
+
+
+def decoded(plan, case, storage):
+    """(ndf, T, Y, X) slab values as float32."""
+    X, Y, T, ndf = case[:4]
+    p, n, yb = plan.slabs()
+    nyb = (Y + yb - 1) // yb
+    a = numpy.empty(ndf * T * nyb * X * yb, numpy.uint16)
+    C.call("gx_memcpy_dtoh", a.ctypes.data, p, a.nbytes, None)
+    if storage == "f16":
+        f = a.view(numpy.float16).astype(numpy.float32)
+    else:
+        f = (a.astype(numpy.uint32) << 16).view(numpy.float32)
+    f = f.reshape(ndf, T, nyb, X, yb)
+    return numpy.moveaxis(f, 4, 3).reshape(ndf, T, nyb * yb, X)[:, :, :Y]
+
+
+@pytest.mark.parametrize("rows", [32, 16])
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("case", CASES)
+def test_matches_oracle_on_its_own_slabs(capi, case, storage, rows):
+    X, Y, T, ndf, Z, W, _, (mn, mx), _ = case
+    plan, sino, angles = plan_of(case, storage)
+    plan.set_tile(rows, "staged")
+    vol = run(plan, case, sino)
+    nrm = numpy.abs(sino).max(axis=(0, 1, 3)).astype(numpy.float32)
+    slabs = decoded(plan, case, storage) * nrm[None, :, None, None]
+    first, last = plan.slab_range()
+    for t in range(T):  # slabs no voxel reads hold anything
+        slabs[:first[t], t] = slabs[last[t] + 1:, t] = 0
+    for y in sorted({0, Y // 3, Y // 2, Y - 1}):
+        s = numpy.ascontiguousarray(slabs[:, :, y])
+        expect = O.project(s if ndf > 1 else s[0], (Z, W), angles,
+                           X / 2.0 - 0.3, 1.0, mn, mx)
+        err = numpy.linalg.norm(vol[y] - expect)
+        assert err <= 1e-5 * numpy.linalg.norm(expect), (y, err)
+    plan.destroy()
+
+
+@pytest.mark.parametrize("case", [CASES[1], CASES[4], CASES[6]])
+def test_exceptional_values_reach_only_their_voxels(capi, case):
+    # A NaN in one row of one tilt makes that filtered row NaN, and the row
+    # it is transformed with (rows 2i and 2i + 1 travel as one complex row):
+    # so are exactly the voxels of the two rows that the tilt sees (an oracle
+    # run of an indicator sinogram shows which); every other voxel keeps its
+    # value.
+    X, Y, T, ndf, Z, W, _, (mn, mx), _ = case
+    plan, sino, angles = plan_of(case, "f16")
+    clean = run(plan, case, sino)
+    assert numpy.isfinite(clean).all()
+    y, t = Y // 2, T // 3
+    broken = sino.copy()
+    broken[y, :, t, X // 2] = numpy.nan
+    vol = run(plan, case, broken)
+    plan.destroy()
+    ones = numpy.zeros((ndf, T, X), numpy.float32)
+    ones[:, t] = 1.0
+    seen = O.project(ones if ndf > 1 else ones[0], (Z, W), angles,
+                     X / 2.0 - 0.3, 1.0, mn, mx) != 0
+    for r in {y, min(y ^ 1, Y - 1)}:
+        numpy.testing.assert_array_equal(numpy.isnan(vol[r]), seen)
+        vol[r][seen] = clean[r][seen]
+    assert numpy.isfinite(vol).all()
+    # the tilt's normalisation may differ (its largest value may have gone)
+    err = numpy.linalg.norm(vol - clean) / numpy.linalg.norm(clean)
+    assert err < 1e-3, err
