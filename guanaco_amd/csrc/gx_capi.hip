@@ -1132,6 +1132,10 @@ int plan_upload(gx_volume_plan *p, hipStream_t s) {
       GX_HIP(launch_bp_mm_windows(p->coef_r.as<float4>(), p->T, p->W, p->Z,
                                   p->dscale, p->doffset, p->ndf,
                                   p->win.as<int2>(), s));
+    else if (p->per_row)  // (its slabs only: the same in every storage)
+      GX_HIP(launch_bp_windows(p->coef.as<float4>(), p->T, p->W, p->Z,
+                               p->dscale, p->doffset, p->ndf,
+                               p->win.as<int2>(), s));
   }
   // the slabs each tilt's voxels read, and the (tilt, defocus) list
   if (p->ndf > 1) {

@@ -1,4 +1,5 @@
-"""The matrix-core backprojector of 16-bit slabs at the edges of its tiles.
+"""The backprojectors of 16-bit slabs at the edges of their tiles: the
+matrix-core kernel, and the kernel for one rotation centre per row.
 
 Each plan's own decoded slabs (times the per-tilt normalisation the filter
 divided out) are backprojected by the FP32 oracle. What is left is the FP32
@@ -126,3 +127,50 @@ def test_exceptional_values_reach_only_their_voxels(capi, case):
     # the tilt's normalisation may differ (its largest value may have gone)
     err = numpy.linalg.norm(vol - clean) / numpy.linalg.norm(clean)
     assert err < 1e-3, err
+
+
+# X, Y, T, ndf, Z, W, (min_df, max_df), drift of the centres (pixels)
+CENTRE_CASES = [
+    # one row; rows past the last block; W no multiple of four
+    (16, 1, 3, 1, 5, 18, (0.0, 0.0), 0.0),
+    (61, 21, 9, 1, 19, 47, (0.0, 0.0), 2.5),
+    # tiles in one slab and across two, centres far off the detector
+    (64, 40, 13, 4, 24, 64, (-64.0, 64.0), 40.0),
+    # more slabs in a tile than the staged kernels hold
+    (64, 33, 7, 16, 16, 36, (-32.0, 32.0), 1.0),
+]
+
+
+@pytest.mark.parametrize("rows", [32, 16])
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("case", CENTRE_CASES)
+def test_centre_per_row_matches_oracle_on_its_own_slabs(capi, case, storage,
+                                                        rows):
+    X, Y, T, ndf, Z, W, (mn, mx), drift = case
+    angles = numpy.deg2rad(numpy.linspace(-60, 60, T)).astype(numpy.float32)
+    rng = numpy.random.default_rng(X + Y)
+    sino = rng.standard_normal((Y, ndf, T, X)).astype(numpy.float32)
+    centres = (X / 2.0 + drift * numpy.linspace(-1, 1, Y)
+               + rng.uniform(-0.5, 0.5, Y)).astype(numpy.float32)
+    if Y == 1:  # (one centre would be a plan without centres)
+        centres = numpy.repeat(centres, 2)
+        sino = numpy.repeat(sino, 2, axis=0)
+        Y = 2
+        case = (X, Y) + case[2:]
+    plan = C.VolumePlan(X, Y, angles, Z, width=W, num_defocus=ndf,
+                        centre=centres, min_defocus=mn, max_defocus=mx,
+                        storage=storage, input_layout=C.INPUT_SINOGRAMS)
+    plan.set_tile(rows, "direct")
+    vol = run(plan, (X, Y, T, ndf, Z, W), sino)
+    nrm = numpy.abs(sino).max(axis=(0, 1, 3)).astype(numpy.float32)
+    slabs = decoded(plan, (X, Y, T, ndf), storage) * nrm[None, :, None, None]
+    first, last = plan.slab_range()
+    for t in range(T):
+        slabs[:first[t], t] = slabs[last[t] + 1:, t] = 0
+    plan.destroy()
+    for y in sorted({0, Y // 2, Y - 1}):
+        s = numpy.ascontiguousarray(slabs[:, :, y])
+        expect = O.project(s if ndf > 1 else s[0], (Z, W), angles,
+                           float(centres[y]), 1.0, mn, mx)
+        err = numpy.linalg.norm(vol[y] - expect)
+        assert err <= 1e-5 * numpy.linalg.norm(expect) + 1e-30, (y, err)
