@@ -1292,15 +1292,15 @@ extern "C" int gx_volume_filter_rows(gx_volume_plan *p, const float *d_in,
                            p->G.as<float2>(), p->Y, p->XB, p->ndf, tc, s,
                            by0, by0 + bny, kr ? kr + t0 : nullptr));
       }
+      const int2 *pl = kr ? p->pairs.as<int2>() + p->pair_off[t0] : nullptr;
+      const int np = kr ? p->pair_off[t0 + tc] - p->pair_off[t0] : 0;
       if (p->rows_bs) {
         GX_HIP(launch_rows_c2r_filter_bs(
             p->G.as<float2>(), p->X, p->Y, p->XB, p->ndf, t0, tc, p->T,
             p->ramp.as<float>(), p->wscale.as<float>(), tmax, p->nrm_mul,
-            p->storage, p->slab.p, p->NYB, p->YB, p->MX, bx, s, by0, bny,
-            kr));
+            p->storage, p->slab.p, p->NYB, p->YB, p->MX, bx, s, by0, bny, pl,
+            np));
       } else {
-        const int2 *pl = kr ? p->pairs.as<int2>() + p->pair_off[t0] : nullptr;
-        const int np = kr ? p->pair_off[t0 + tc] - p->pair_off[t0] : 0;
         GX_HIP(launch_rows_c2r_filter(
             p->G.as<float2>(), p->X, p->Y, p->XB, p->ndf, t0, tc, p->T,
             p->wscale.as<float>(), tmax, p->nrm_mul,

@@ -589,7 +589,8 @@ __global__ __launch_bounds__(2 * (2 * X / default_e(2 * X))) void
 }
 
 // Writes a row group of the slab: P slots, slot p holding rows (R0 + 2p,
-// R0 + 2p + 1) of column tid + m NT in out[m] (E = X / NT per thread), of
+// R0 + 2p + 1) of column tid + m NT in out[m] (E = X / NT per thread, the
+// slot's LDS region at least fft_lds_len(X, E)), of
 // which the first ncols columns are stored ([y / YB][x][y % YB], rows of
 // ncols). s: the workgroup's P slot regions of fft_lds_len(X, E) float2.
 // One slot, and the last, partial row group, store from registers; otherwise
@@ -598,12 +599,11 @@ __global__ __launch_bounds__(2 * (2 * X / default_e(2 * X))) void
 // banks), in NCH passes of XC columns when the regions do not hold all X
 // columns at once, and the workgroup writes each column's RB = 2P rows as
 // whole 4-, 8- or 16-byte runs.
-template <int X, int STORE, int P>
+template <int X, int STORE, int P, int E = default_e(X)>
 __device__ __forceinline__ void store_row_group(
-    const typename RowPair<STORE>::T (&out)[default_e(X)], float2 *s, int p,
+    const typename RowPair<STORE>::T (&out)[E], float2 *s, int p,
     int tid, typename StoreT<STORE>::T *__restrict__ slab, int k, int t,
     int R0, int Y, int ncols, int T, int NYB, int YB) {
-  constexpr int E = default_e(X);
   constexpr int NT = X / E;
   using PT = typename RowPair<STORE>::T;
   using ST = typename StoreT<STORE>::T;
@@ -1128,11 +1128,21 @@ __global__ void k_absmax_rows(const float *__restrict__ src, size_t st,
 // spectra are computed in FP64 on the host (m^2 mod 2n in integers) and
 // rounded once.
 // v[m] holds x[tid + m NT] for tid + m NT < n (anything beyond is ignored);
-// on return v[m] = X[tid + m NT] for indices < n and 0 beyond.
-template <int M, int E, int DIR, int LS>
+// on return v[m] = X[tid + m NT] for indices < n and 0 beyond. n <= M / 2, so
+// the values from m = E / 2 on are zero before the first transform, which
+// skips adding them. (The chirp products stay in branches, and the second
+// transform computes all its outputs: the compiler chooses which product of
+// a complex multiplication to fuse from what surrounds it, and other forms
+// changed the last bits of the result, and with them the rounding of 16-bit
+// slabs.) A row's transform that lies within one wave synchronises only that
+// wave.
+constexpr bool bs_wave(int M, int LS) {
+  return LS == 1 && M / default_e(M) <= 64;
+}
+template <int M, int E, int DIR, int LS, bool WAVE = bs_wave(M, LS)>
 __device__ __forceinline__ void bluestein(
     float2 (&v)[E], float2 *lds, int tid,
-    const typename Fft<M, E, -1, LS>::Twiddles &tw, const BluesteinTable &b) {
+    const FftTwiddles<M, E> &tw, const BluesteinTable &b) {
   constexpr int NT = M / E;
 #pragma unroll
   for (int m = 0; m < E; ++m) {
@@ -1144,11 +1154,11 @@ __device__ __forceinline__ void bluestein(
       v[m] = make_float2(0.0f, 0.0f);
     }
   }
-  Fft<M, E, -1, LS>::run(v, lds, tid, tw);
+  Fft<M, E, -1, LS, WAVE>::template run<true>(v, lds, tid, tw);
   const float2 *B = DIR < 0 ? b.bf : b.bi;
 #pragma unroll
   for (int m = 0; m < E; ++m) v[m] = cmul(v[m], B[tid + m * NT]);
-  Fft<M, E, 1, LS>::run(v, lds, tid, tw);
+  Fft<M, E, 1, LS, WAVE>::run(v, lds, tid, tw);
 #pragma unroll
   for (int m = 0; m < E; ++m) {
     const int j = tid + m * NT;
@@ -1161,10 +1171,11 @@ __device__ __forceinline__ void bluestein(
   }
 }
 
-// Bluestein row passes: P row pairs per workgroup, one M-point slot each
-// (P = 2; P = 1 at M = 16384, whose slot is a whole 1024-thread workgroup
-// with 139 KB of LDS).
-constexpr int bs_row_slots(int M) { return M >= 16384 ? 1 : 2; }
+// Bluestein row passes: P row pairs per workgroup, one M-point slot each: 2
+// up to 2048 points, 1 from 4096 on (at 4096, two slots made a workgroup of
+// 512 threads with 167 registers, of which a CU holds one, two waves per
+// SIMD; of one-slot workgroups it holds three).
+constexpr int bs_row_slots(int M) { return M >= 4096 ? 1 : 2; }
 
 // Pass 1 for any X: rows (ya, yb) as one complex row, forward X-point DFT,
 // then the Hermitian split into the two half spectra (as k_rows_r2c).
@@ -1223,21 +1234,29 @@ __global__ __launch_bounds__(P * (M / default_e(M))) void k_rows_r2c_bs(
 
 // Pass 2 for any Y: CW of the CB columns of a block per workgroup (LDS
 // holds CW M-point transforms), forward Y-point DFT, then per defocus the
-// flip and the inverse Y-point DFT.
+// flip and the inverse Y-point DFT. The grid is 1D over (column part, tilt,
+// column block), XCD-remapped as k_cols' is. At 2048 points a workgroup is
+// 512 threads, and a CU holds two only within 128 registers (12 spilled;
+// with 164 it held one: 41 tilts of 960 x 928, 4 slabs, 0.95 -> 0.63 ms).
 template <int M, int CW>
-__global__ __launch_bounds__(CW *(M / default_e(M))) void k_cols_bs(
+__global__ __launch_bounds__(CW *(M / default_e(M)))
+__attribute__((amdgpu_waves_per_eu(M == 2048 || M == 16384 ? 4 : M <= 1024 ? 3 : 2))) void
+    k_cols_bs(
     const float2 *__restrict__ F, const int8_t *__restrict__ mask,
     float2 *__restrict__ G, int Y, int XB, int ndf,
     const float2 *__restrict__ tw, BluesteinTable by, int ylo, int yhi,
     const int2 *__restrict__ krange) {
   constexpr int E = default_e(M);
   constexpr int NT = M / E;
+  constexpr int H = CB / CW;  // workgroups per column block
   static_assert(CB % CW == 0, "column groups split a block");
   __shared__ float2 s[fft_lds_len(M, E) * CW];
   const int c = threadIdx.x % CW, tid = threadIdx.x / CW;
-  const int cb = blockIdx.x / (CB / CW);
-  const int ci = (blockIdx.x % (CB / CW)) * CW + c;
-  const int t = blockIdx.y;
+  const unsigned lb = xcd_remap(blockIdx.x, gridDim.x);
+  const unsigned nt = gridDim.x / (H * (unsigned)XB);  // tilts of the launch
+  const int ci = (int)(lb % H) * CW + c;
+  const int t = (int)((lb / H) % nt);
+  const int cb = (int)(lb / (H * nt));
   const float2 *src = F + ((size_t)t * XB + cb) * Y * CB;
   typename Fft<M, E, -1, CW>::Twiddles twm;
   twm.load(tid, tw);
@@ -1245,7 +1264,7 @@ __global__ __launch_bounds__(CW *(M / default_e(M))) void k_cols_bs(
 #pragma unroll
   for (int m = 0; m < E; ++m) {
     const int y = tid + m * NT;
-    v[m] = y < Y ? src[(size_t)y * CB + ci] : make_float2(0.0f, 0.0f);
+    v[m] = m < E / 2 ? src[(size_t)min(y, Y - 1) * CB + ci] : make_float2(0.0f, 0.0f);
   }
   bluestein<M, E, -1, CW>(v, s + c, tid, twm, by);
   const int2 kr = krange != nullptr ? krange[t] : make_int2(0, ndf - 1);
@@ -1259,7 +1278,7 @@ __global__ __launch_bounds__(CW *(M / default_e(M))) void k_cols_bs(
 #pragma unroll
     for (int m = 0; m < E; ++m) {
       const int y = tk + m * NT;
-      const float f = y < Y ? mask_value(mk[(size_t)y * CB + ck]) : 0.0f;
+      const float f = m < E / 2 ? mask_value(mk[(size_t)min(y, Y - 1) * CB + ck]) : 0.0f;
       w[m] = make_float2(v[m].x * f, v[m].y * f);
     }
     typename Fft<M, E, -1, CW>::Twiddles twk;
@@ -1290,11 +1309,10 @@ __global__ __launch_bounds__(P * (M / default_e(M))) void k_rows_c2r_bs(
   twm.load(tid, tw);
   float2 v[E];
 #pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const int n = tid + m * NT;
-    v[m] = n < X ? load_pair_spectrum(g, X, Y, ya, yb, n)
-                 : make_float2(0.0f, 0.0f);
-  }
+  for (int m = 0; m < E / 2; ++m)
+    v[m] = load_pair_spectrum(g, X, Y, ya, yb, min(tid + m * NT, X - 1));
+#pragma unroll
+  for (int m = E / 2; m < E; ++m) v[m] = make_float2(0.0f, 0.0f);
   bluestein<M, E, 1, 1>(v, s[p], tid, twm, bx);
   float *o = out + ((size_t)tl * ndf + k) * Y * X;
 #pragma unroll
@@ -1310,8 +1328,23 @@ __global__ __launch_bounds__(P * (M / default_e(M))) void k_rows_c2r_bs(
 // Pass 3 for any X, fused with the ramp filter: the corrected rows (X
 // samples, unnormalised inverse) are zero-padded to M >= 2X - 1 and filtered
 // with the truncated-kernel ramp table, as k_filter_rows does for real rows.
-template <int M, int STORE, int P = bs_row_slots(M)>
-__global__ __launch_bounds__(P * (M / default_e(M))) void
+// Grid and slab stores as in k_rows_c2r_ramp: 1D over (row group, listed
+// (tilt, defocus) pair or every one), XCD-remapped so that the halves of the
+// spectrum lines and slab runs that row groups share meet in one L2; the P
+// slots of a workgroup (2P rows, dividing the slab's row blocking) stage
+// their rows in LDS and leave as whole runs. Bound by vector issue (four
+// M-point transforms per row pair): 90 tilts of 1500 x 200, 8 slabs, FP32
+// (M = 4096) 2.53 -> 1.4 ms; 41 tilts of 960 x 928, 4 slabs, FP16 (M = 2048)
+// 1.15 -> 0.75 ms against a grid of every pair, 2- and 4-byte stores and two
+// slots at every length.
+constexpr int bs_filter_slots(int M) {
+  // (one at 8 points, where a thread has one column and F32 staging takes
+  // two passes of half the columns)
+  return M <= 8 ? 1 : M <= 1024 ? 4 : M == 2048 ? 2 : 1;
+}
+template <int M, int STORE, int P>
+__global__ __launch_bounds__(P * (M / default_e(M)))
+__attribute__((amdgpu_waves_per_eu(M >= 16384 ? 4 : M >= 8192 ? 2 : 3))) void
     k_rows_c2r_filter_bs(const float2 *__restrict__ G, int X, int Y, int XB,
                          int ndf, int t0, int T,
                          const float *__restrict__ ramp,
@@ -1320,46 +1353,55 @@ __global__ __launch_bounds__(P * (M / default_e(M))) void
                          typename StoreT<STORE>::T *__restrict__ slab,
                          int NYB, int YB, const float2 *__restrict__ tw,
                          BluesteinTable bx, int y0, int ny,
-                         const int2 *__restrict__ krange) {
+                         const int2 *__restrict__ pairs) {
   constexpr int E = default_e(M);
   constexpr int NT = M / E;
-  __shared__ float2 s[P][fft_lds_len(M, E)];
+  constexpr int SL = fft_lds_len(M, E);
+  using PT = typename RowPair<STORE>::T;
+  __shared__ float2 s[P * SL];
   const int p = threadIdx.x / NT, tid = threadIdx.x % NT;
-  const int k = blockIdx.y, tl = blockIdx.z, t = t0 + tl;
-  if (krange != nullptr && (k < krange[t].x || k > krange[t].y)) return;
-  // band-relative rows ra, rb of the slab; spectrum rows y0 + ra, y0 + rb
-  const int ra = blockIdx.x * (2 * P) + 2 * p, rb = ra + 1;
-  const int ya = y0 + ra, yb = ya + 1;
+  const unsigned nry = (unsigned)(ny + 2 * P - 1) / (2 * P);
+  const unsigned lb = xcd_remap(blockIdx.x, gridDim.x);
+  int k, tl;
+  if (pairs != nullptr) {
+    const int2 pk = pairs[lb / nry];
+    tl = pk.x - t0;
+    k = pk.y;
+  } else {
+    k = (int)((lb / nry) % (unsigned)ndf);
+    tl = (int)(lb / (nry * (unsigned)ndf));
+  }
+  const int t = t0 + tl;
+  // band-relative rows R0 .. of the slab; spectrum rows y0 + R0 ..
+  const int R0 = (int)(lb % nry) * (2 * P);
+  const int ya = y0 + R0 + 2 * p, yb = ya + 1;
   const float2 *g = G + ((size_t)tl * ndf + k) * XB * Y * CB;
+  float2 *ls = s + p * SL;
   typename Fft<M, E, -1, 1>::Twiddles twm;
   twm.load(tid, tw);
   float2 v[E];
 #pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const int n = tid + m * NT;
-    v[m] = n < X ? load_pair_spectrum(g, X, Y, ya, yb, n)
-                 : make_float2(0.0f, 0.0f);
-  }
-  bluestein<M, E, 1, 1>(v, s[p], tid, twm, bx);  // zero beyond X
-  Fft<M, E, -1, 1>::run(v, s[p], tid, twm);
+  for (int m = 0; m < E / 2; ++m)
+    v[m] = load_pair_spectrum(g, X, Y, ya, yb, min(tid + m * NT, X - 1));
+#pragma unroll
+  for (int m = E / 2; m < E; ++m) v[m] = make_float2(0.0f, 0.0f);
+  bluestein<M, E, 1, 1>(v, ls, tid, twm, bx);  // zero beyond X
+  Fft<M, E, -1, 1, bs_wave(M, 1)>::template run<true>(v, ls, tid, twm);
 #pragma unroll
   for (int m = 0; m < E; ++m) {
     const int j = tid + m * NT;
     const float r = ramp[j <= M / 2 ? j : M - j];
     v[m] = make_float2(v[m].x * r, v[m].y * r);
   }
-  Fft<M, E, 1, 1>::run(v, s[p], tid, twm);
+  Fft<M, E, 1, 1, bs_wave(M, 1)>::run(v, ls, tid, twm);
   const float sc =
       wscale[t] * (STORE == kF32 ? 1.0f : inv_norm(tmax, t, nrm_mul));
-  using ST = StoreT<STORE>;
+  PT out[E / 2];
 #pragma unroll
-  for (int m = 0; m < E; ++m) {
-    const int n = tid + m * NT;
-    if (n < X) {
-      if (ra < ny) slab[slab_index(k, t, ra, n, T, NYB, X, YB)] = ST::pack(v[m].x * sc);
-      if (rb < ny) slab[slab_index(k, t, rb, n, T, NYB, X, YB)] = ST::pack(v[m].y * sc);
-    }
-  }
+  for (int m = 0; m < E / 2; ++m)
+    out[m] = RowPair<STORE>::pack(v[m].x * sc, v[m].y * sc);
+  store_row_group<M / 2, STORE, P, E / 2>(out, s, p, tid, slab, k, t, R0, ny,
+                                          X, T, NYB, YB);
 }
 
 // ------------------------------------------------------------ launchers ---
@@ -1883,7 +1925,7 @@ hipError_t launch_cols_bs(const float2 *F, const int8_t *mask, float2 *G,
   switch (M) {
 #define C_(n)                                                                 \
   case n:                                                                     \
-    hipLaunchKernelGGL((k_cols_bs<n, CB>), dim3(XB, ntilts),                  \
+    hipLaunchKernelGGL((k_cols_bs<n, CB>), dim3(XB * ntilts),                 \
                        dim3(CB * (n / default_e(n))), 0, s, F, mask, G, Y,    \
                        XB, ndf, tw, by, ylo, yhi, krange);                    \
     break;
@@ -1891,7 +1933,7 @@ hipError_t launch_cols_bs(const float2 *F, const int8_t *mask, float2 *G,
 #undef C_
 #define C_(n)                                                                 \
   case n:                                                                     \
-    hipLaunchKernelGGL((k_cols_bs<n, 1>), dim3(XB * CB, ntilts),              \
+    hipLaunchKernelGGL((k_cols_bs<n, 1>), dim3(XB * CB * ntilts),             \
                        dim3(n / default_e(n)), 0, s, F, mask, G, Y, XB, ndf,  \
                        tw, by, ylo, yhi, krange);                             \
     break;
@@ -1926,6 +1968,22 @@ hipError_t launch_rows_c2r_bs(const float2 *G, int X, int Y, int XB, int ndf,
   return hipGetLastError();
 }
 
+template <int M, int STORE, int P>
+static void launch_c2r_filter_bs_p(unsigned nb, const float2 *G, int X, int Y,
+                                   int XB, int ndf, int t0, int T,
+                                   const float *ramp, const float *wscale,
+                                   const uint32_t *tmax, float nrm_mul,
+                                   void *slab, int NYB, int YB,
+                                   const BluesteinTable &bx, hipStream_t s,
+                                   const float2 *tw, int y0, int ny,
+                                   const int2 *pairs) {
+  using ST = typename StoreT<STORE>::T;
+  hipLaunchKernelGGL((k_rows_c2r_filter_bs<M, STORE, P>), dim3(nb),
+                     dim3(P * (M / default_e(M))), 0, s, G, X, Y, XB, ndf, t0,
+                     T, ramp, wscale, tmax, nrm_mul, (ST *)slab, NYB, YB, tw,
+                     bx, y0, ny, pairs);
+}
+
 template <int STORE>
 static hipError_t launch_c2r_filter_bs_t(const float2 *G, int X, int Y,
                                          int XB, int ndf, int t0, int ntilts,
@@ -1935,17 +1993,20 @@ static hipError_t launch_c2r_filter_bs_t(const float2 *G, int X, int Y,
                                          void *slab, int NYB, int YB, int M,
                                          const BluesteinTable &bx,
                                          hipStream_t s, const float2 *tw,
-                                         int y0, int ny, const int2 *krange) {
-  using ST = typename StoreT<STORE>::T;
+                                         int y0, int ny, const int2 *pairs,
+                                         int npairs) {
   switch (M) {
 #define C_(n)                                                                  \
   case n: {                                                                    \
-    constexpr int P = bs_row_slots(n);                                         \
-    const dim3 grid((ny + 2 * P - 1) / (2 * P), ndf, ntilts);                  \
-    hipLaunchKernelGGL((k_rows_c2r_filter_bs<n, STORE>), grid,                 \
-                       dim3(P * (n / default_e(n))), 0, s, G, X, Y, XB, ndf,   \
-                       t0, T, ramp, wscale, tmax, nrm_mul, (ST *)slab, NYB, YB, \
-                       tw, bx, y0, ny, krange);                                \
+    constexpr int P = bs_filter_slots(n);                                      \
+    if (YB % (2 * P) != 0) return hipErrorInvalidValue;                        \
+    const size_t nb = (size_t)((ny + 2 * P - 1) / (2 * P)) *                   \
+                      (pairs ? (size_t)npairs : (size_t)ndf * ntilts);         \
+    if (nb == 0) return hipSuccess;                                            \
+    if (nb > 0xffffffffu) return hipErrorInvalidValue;                         \
+    launch_c2r_filter_bs_p<n, STORE, P>((unsigned)nb, G, X, Y, XB, ndf, t0, T, \
+                                        ramp, wscale, tmax, nrm_mul, slab,     \
+                                        NYB, YB, bx, s, tw, y0, ny, pairs);    \
     break;                                                                     \
   }
     GX_BS_CASES(C_)
@@ -1963,14 +2024,14 @@ hipError_t launch_rows_c2r_filter_bs(const float2 *G, int X, int Y, int XB,
                                      int store, void *slab, int NYB, int YB,
                                      int M, const BluesteinTable &bx,
                                      hipStream_t s, int y0, int ny,
-                                     const int2 *krange) {
+                                     const int2 *pairs, int npairs) {
   hipError_t err;
   const float2 *tw = twiddles(&err);
   if (err != hipSuccess) return err;
   if (ny < 0) ny = Y - y0;
   if (y0 < 0 || y0 % YB != 0 || ny <= 0 || y0 + ny > Y)
     return hipErrorInvalidValue;
-#define A_ G, X, Y, XB, ndf, t0, ntilts, T, ramp, wscale, tmax, nrm_mul, slab, NYB, YB, M, bx, s, tw, y0, ny, krange
+#define A_ G, X, Y, XB, ndf, t0, ntilts, T, ramp, wscale, tmax, nrm_mul, slab, NYB, YB, M, bx, s, tw, y0, ny, pairs, npairs
   switch (store) {
     case kF32:
       return launch_c2r_filter_bs_t<kF32>(A_);

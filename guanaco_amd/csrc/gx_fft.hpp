@@ -102,7 +102,20 @@ __host__ __device__ __forceinline__ float2 rot16(float2 a) {
   }
 }
 
-template <int R, int DIR>
+// dft4 with a2 = a3 = 0 (the same values, without adding the zeros).
+template <int DIR>
+__host__ __device__ __forceinline__ void dft4_low(float2 &a0, float2 &a1,
+                                                  float2 &a2, float2 &a3) {
+  const float2 t0 = a0, t2 = a1, t3 = mul_i<DIR>(a1);
+  a0 = cadd(t0, t2);
+  a2 = csub(t0, t2);
+  a1 = cadd(t0, t3);
+  a3 = csub(t0, t3);
+}
+
+// LOW: the upper half of the inputs is zero (R = 16 skips the additions of
+// those zeros; other radices add them).
+template <int R, int DIR, bool LOW = false>
 __host__ __device__ __forceinline__ void dft(float2 *v) {
   #pragma clang fp contract(fast)
   if constexpr (R == 1) {
@@ -135,7 +148,10 @@ __host__ __device__ __forceinline__ void dft(float2 *v) {
 #pragma unroll
     for (int n2 = 0; n2 < 4; ++n2) {
       float2 a0 = v[n2], a1 = v[n2 + 4], a2 = v[n2 + 8], a3 = v[n2 + 12];
-      dft4<DIR>(a0, a1, a2, a3);
+      if constexpr (LOW)
+        dft4_low<DIR>(a0, a1, a2, a3);
+      else
+        dft4<DIR>(a0, a1, a2, a3);
       b[n2 * 4 + 0] = a0;
       b[n2 * 4 + 1] = a1;
       b[n2 * 4 + 2] = a2;
@@ -417,14 +433,20 @@ struct Fft {
   }
 
   // In: v[m] = x[tid + m*NT]. Out: v[m] = X[tid + m*NT]. lds holds kLds * LS
-  // float2 (only every LS-th used). Returns with lds free for reuse.
+  // float2 (only every LS-th used). Returns with lds free for reuse. LOW:
+  // x is zero from N / 2 on (v[m] for m >= E / 2 is not read).
+  template <bool LOW = false>
   __device__ __forceinline__ static void run(float2 (&v)[E], float2 *lds,
                                              int tid, const Twiddles &tw) {
     #pragma clang fp contract(fast)
+    if constexpr (LOW && E != 16) {
+#pragma unroll
+      for (int m = E / 2; m < E; ++m) v[m] = make_float2(0.0f, 0.0f);
+    }
     if constexpr (NS == 1) {
-      dft<E, DIR>(v);
+      dft<E, DIR, LOW>(v);
     } else {
-      dft<E, DIR>(v);
+      dft<E, DIR, LOW>(v);
 #pragma unroll
       for (int m = 0; m < E; ++m) lds[(tid * (E + 1) + m) * LS] = v[m];
       fft_sync<WAVE>();

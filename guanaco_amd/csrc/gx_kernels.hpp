@@ -83,7 +83,8 @@ hipError_t launch_rows_c2r_filter_bs(const float2 *G, int X, int Y, int XB,
                                      int store, void *slab, int NYB, int YB,
                                      int M, const BluesteinTable &bx,
                                      hipStream_t s, int y0 = 0, int ny = -1,
-                                     const int2 *krange = nullptr);
+                                     const int2 *pairs = nullptr,
+                                     int npairs = 0);
 
 // CTF parameters in the reference's units (ctf.h:167-178): A and rad
 struct CtfParams {
