@@ -122,6 +122,16 @@ class CtfDesc(ctypes.Structure):
                 ("recentre", _int), ("gpu_index", _int)]
 
 
+class StackDesc(ctypes.Structure):
+    _fields_ = [("num_pixels", _sz), ("num_rows", _sz), ("num_images", _sz),
+                ("num_defocus", _sz),
+                ("defocus", ctypes.POINTER(ctypes.c_double)),
+                ("pixel_size", ctypes.c_double),
+                ("wavelength", ctypes.c_double), ("Cs", ctypes.c_double),
+                ("Ca", ctypes.c_double), ("Pa", ctypes.c_double),
+                ("phi", ctypes.c_double), ("gpu_index", _int)]
+
+
 class TuneEntry(ctypes.Structure):
     _fields_ = [("kind", _int), ("rows", _int), ("filter_ms", ctypes.c_float),
                 ("bp_ms", ctypes.c_float)]
@@ -171,6 +181,7 @@ SIGNATURES = {
     "gx_project": [ctypes.POINTER(ReconCfg), _f32p, _f32p],
     "gx_filter": [_f32p, _f32p, _sz, _sz, _int],
     "gx_corr": [_f32p, _f32p, _f32p, _sz, _sz, _sz, _int],
+    "gx_correct_stack": [ctypes.POINTER(StackDesc), _f32p, _f32p],
     "gx_volume_plan_bytes": [ctypes.POINTER(VolumeDesc), ctypes.POINTER(_sz)],
     "gx_volume_plan_create": [ctypes.POINTER(VolumeDesc), ctypes.POINTER(_vp)],
     "gx_volume_plan_destroy": [_vp],

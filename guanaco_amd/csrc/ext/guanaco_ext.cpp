@@ -71,6 +71,28 @@ void corr(const py::array_t<float> &image,
   guanaco::correct(im, c, r, xsize, ysize, num_ctf, device);
 }
 
+// Additive: corr() of a stack of images (T, Y, X) with the CTF `ctf` at each
+// absolute defocus (its own df is not read), evaluated on the device, into
+// out (T, ndf, Y, X), which is written in place.
+void correct_stack(const py::array_t<float, py::array::c_style> &images,
+                   py::array_t<float, py::array::c_style> &out,
+                   const std::vector<double> &defocus, const guanaco::CTF &ctf,
+                   double pixel_size, eDevice device, int gpu_index) {
+  GUANACO_ASSERT(images.ndim() == 3);
+  GUANACO_ASSERT(out.ndim() == 4);
+  GUANACO_ASSERT(out.shape()[0] == images.shape()[0]);
+  GUANACO_ASSERT(out.shape()[1] == (py::ssize_t)defocus.size());
+  GUANACO_ASSERT(out.shape()[2] == images.shape()[1]);
+  GUANACO_ASSERT(out.shape()[3] == images.shape()[2]);
+  const float *in = images.data();
+  float *o = out.mutable_data();
+  const std::size_t T = images.shape()[0], Y = images.shape()[1],
+                    X = images.shape()[2];
+  py::gil_scoped_release release;
+  guanaco::correct_stack(in, T, X, Y, defocus, ctf, pixel_size, o, device,
+                         gpu_index);
+}
+
 py::array_t<std::complex<double>> ctf_simple_wh(const guanaco::CTF &c,
                                                 std::size_t w, std::size_t h,
                                                 double ps) {
@@ -367,6 +389,10 @@ PYBIND11_MODULE(guanaco_ext, m) {
   // ext/correct.h:71-76
   m.def("corr", &corr, py::arg("image"), py::arg("ctf"), py::arg("rec"),
         py::arg("device") = guanaco::e_host);
+
+  m.def("correct_stack", &correct_stack, py::arg("images"),
+        py::arg("out").noconvert(), py::arg("defocus"), py::arg("ctf"),
+        py::arg("pixel_size"), py::arg("device"), py::arg("gpu_index") = -1);
 
   // ext/reconstruct.h:88-101
   m.def("recon", &recon, py::arg("sinogram"), py::arg("reconstruction"),

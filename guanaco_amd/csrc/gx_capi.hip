@@ -690,6 +690,60 @@ static int check_pow2_corr_sizes(size_t X, size_t Y) {
   return GX_OK;
 }
 
+namespace {
+
+// Transform tables of a standalone correction.
+struct CorrTables {
+  bool rows = false, cols = false;  // power-of-two transforms
+  size_t MX = 0, MY = 0;
+  DevBuf tab;
+  gx::BluesteinTable bx{}, by{};
+  int create(size_t X, size_t Y) {
+    rows = rows_pow2(X);
+    cols = cols_pow2(Y);
+    MX = filter_length(X);
+    MY = filter_length(Y);
+    std::vector<float2> h;
+    if (!rows) bluestein_tables(X, MX, h);
+    const size_t y0 = h.size();
+    if (!cols) bluestein_tables(Y, MY, h);
+    if (!h.empty()) {
+      GX_HIP(tab.alloc(sizeof(float2) * h.size()));
+      GX_HIP(hipMemcpy(tab.p, h.data(), sizeof(float2) * h.size(),
+                       hipMemcpyHostToDevice));
+    }
+    bx = bluestein_view(tab.as<float2>(), X, MX);
+    by = bluestein_view(tab.as<float2>() + y0, Y, MY);
+    return GX_OK;
+  }
+};
+
+// n images (device) through the three passes: out[image][defocus][y][x].
+int correct_images(const CorrTables &t, const float *img, int X, int Y, int XB,
+                   int ndf, int n, const int8_t *mask, float2 *F, float2 *G,
+                   float *out, hipStream_t s) {
+  const size_t npix = (size_t)X * Y;
+  if (t.rows) {
+    GX_HIP(launch_rows_r2c(img, npix, X, Y, XB, n, F, nullptr, 0, s));
+  } else {
+    GX_HIP(launch_rows_r2c_bs(img, npix, X, Y, XB, n, F, nullptr, 0, (int)t.MX,
+                              t.bx, s));
+  }
+  if (t.cols) {
+    GX_HIP(launch_cols(F, mask, G, Y, XB, ndf, n, s));
+  } else {
+    GX_HIP(launch_cols_bs(F, mask, G, Y, XB, ndf, n, (int)t.MY, t.by, s));
+  }
+  if (t.rows) {
+    GX_HIP(launch_rows_c2r(G, X, Y, XB, ndf, n, out, s));
+  } else {
+    GX_HIP(launch_rows_c2r_bs(G, X, Y, XB, ndf, n, out, (int)t.MX, t.bx, s));
+  }
+  return GX_OK;
+}
+
+}  // namespace
+
 extern "C" int gx_corr(const float *image, const float *ctf, float *rec,
                        size_t xsize, size_t ysize, size_t num_ctf,
                        int gpu_index) {
@@ -717,47 +771,71 @@ extern "C" int gx_corr(const float *image, const float *ctf, float *rec,
   GX_HIP(hipMemcpy(d_ctf.p, ctf, sizeof(float2) * npix * num_ctf,
                    hipMemcpyHostToDevice));
   hipStream_t s = nullptr;
-  const bool rp = rows_pow2(xsize), cp = cols_pow2(ysize);
-  const size_t MX = filter_length(xsize), MY = filter_length(ysize);
-  std::vector<float2> tab;
-  if (!rp) bluestein_tables(xsize, MX, tab);
-  const size_t ytab = tab.size();
-  if (!cp) bluestein_tables(ysize, MY, tab);
-  DevBuf d_tab;
-  if (!tab.empty()) {
-    GX_HIP(d_tab.alloc(sizeof(float2) * tab.size()));
-    GX_HIP(hipMemcpy(d_tab.p, tab.data(), sizeof(float2) * tab.size(),
-                     hipMemcpyHostToDevice));
-  }
-  const gx::BluesteinTable bx = bluestein_view(d_tab.as<float2>(), xsize, MX);
-  const gx::BluesteinTable by =
-      bluestein_view(d_tab.as<float2>() + ytab, ysize, MY);
+  CorrTables tab;
+  rc = tab.create(xsize, ysize);
+  if (rc) return rc;
   GX_HIP(launch_mask_from_ctf(d_mask.as<int8_t>(), d_ctf.as<float2>(), X, Y, XB,
-                              ndf, cp, s));
-  if (rp) {
-    GX_HIP(launch_rows_r2c(d_img.as<float>(), npix, X, Y, XB, 1,
-                           d_F.as<float2>(), nullptr, 0, s));
-  } else {
-    GX_HIP(launch_rows_r2c_bs(d_img.as<float>(), npix, X, Y, XB, 1,
-                              d_F.as<float2>(), nullptr, 0, (int)MX, bx, s));
-  }
-  if (cp) {
-    GX_HIP(launch_cols(d_F.as<float2>(), d_mask.as<int8_t>(),
-                       d_G.as<float2>(), Y, XB, ndf, 1, s));
-  } else {
-    GX_HIP(launch_cols_bs(d_F.as<float2>(), d_mask.as<int8_t>(),
-                          d_G.as<float2>(), Y, XB, ndf, 1, (int)MY, by, s));
-  }
-  if (rp) {
-    GX_HIP(launch_rows_c2r(d_G.as<float2>(), X, Y, XB, ndf, 1,
-                           d_out.as<float>(), s));
-  } else {
-    GX_HIP(launch_rows_c2r_bs(d_G.as<float2>(), X, Y, XB, ndf, 1,
-                              d_out.as<float>(), (int)MX, bx, s));
-  }
+                              ndf, tab.cols, s));
+  rc = correct_images(tab, d_img.as<float>(), X, Y, XB, ndf, 1,
+                      d_mask.as<int8_t>(), d_F.as<float2>(), d_G.as<float2>(),
+                      d_out.as<float>(), s);
+  if (rc) return rc;
   GX_HIP(hipStreamSynchronize(s));
   GX_HIP(hipMemcpy(rec, d_out.p, sizeof(float) * npix * num_ctf,
                    hipMemcpyDeviceToHost));
+  return GX_OK;
+}
+
+extern "C" int gx_correct_stack(const gx_stack_desc *d, const float *images,
+                                float *out) {
+  GX_CHECK(d != nullptr && images != nullptr && out != nullptr);
+  GX_CHECK(d->num_pixels > 0 && d->num_rows > 0);
+  GX_CHECK(d->num_images > 0 && d->num_defocus > 0);
+  GX_CHECK(d->defocus != nullptr);
+  GX_CHECK(d->pixel_size > 0);
+  int rc = check_corr_sizes(d->num_pixels, d->num_rows);
+  if (rc) return rc;
+  rc = select_device(d->gpu_index);
+  if (rc) return rc;
+  const int X = (int)d->num_pixels, Y = (int)d->num_rows;
+  const int ndf = (int)d->num_defocus;
+  const int XB = X / 2 / CB + 1;
+  const size_t npix = d->num_pixels * d->num_rows;
+  const size_t nspec = (size_t)XB * CB * Y;
+  // images per launch: about 512 MiB of spectra and results
+  const size_t each = sizeof(float) * npix * (1 + d->num_defocus) +
+                      sizeof(float2) * nspec * (1 + d->num_defocus);
+  const size_t n =
+      std::min(d->num_images, std::max<size_t>(1, ((size_t)512 << 20) / each));
+  DevBuf d_img, d_df, d_mask, d_F, d_G, d_out;
+  GX_HIP(d_img.alloc(sizeof(float) * npix * n));
+  GX_HIP(d_df.alloc(sizeof(double) * d->num_defocus));
+  GX_HIP(d_mask.alloc(nspec * d->num_defocus));
+  GX_HIP(d_F.alloc(sizeof(float2) * nspec * n));
+  GX_HIP(d_G.alloc(sizeof(float2) * nspec * d->num_defocus * n));
+  GX_HIP(d_out.alloc(sizeof(float) * npix * d->num_defocus * n));
+  hipStream_t s = nullptr;
+  CorrTables tab;
+  rc = tab.create(d->num_pixels, d->num_rows);
+  if (rc) return rc;
+  GX_HIP(hipMemcpy(d_df.p, d->defocus, sizeof(double) * d->num_defocus,
+                   hipMemcpyHostToDevice));
+  GX_HIP(launch_ctf_mask(d_mask.as<int8_t>(), X, Y, XB, ndf,
+                         d_df.as<double>(), d->wavelength, d->Cs, d->Ca, d->Pa,
+                         d->phi, d->pixel_size, tab.cols, s));
+  for (size_t i = 0; i < d->num_images; i += n) {
+    const size_t m = std::min(n, d->num_images - i);
+    GX_HIP(hipMemcpy(d_img.p, images + i * npix, sizeof(float) * npix * m,
+                     hipMemcpyHostToDevice));
+    rc = correct_images(tab, d_img.as<float>(), X, Y, XB, ndf, (int)m,
+                        d_mask.as<int8_t>(), d_F.as<float2>(),
+                        d_G.as<float2>(), d_out.as<float>(), s);
+    if (rc) return rc;
+    GX_HIP(hipStreamSynchronize(s));
+    GX_HIP(hipMemcpy(out + i * npix * d->num_defocus, d_out.p,
+                     sizeof(float) * npix * d->num_defocus * m,
+                     hipMemcpyDeviceToHost));
+  }
   return GX_OK;
 }
 

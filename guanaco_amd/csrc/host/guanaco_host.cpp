@@ -82,6 +82,28 @@ void correct(const float *image, const std::complex<float> *ctf, float *rec,
                        ysize, num_ctf, gpu_index));
 }
 
+void correct_stack(const float *images, std::size_t num_images,
+                   std::size_t xsize, std::size_t ysize,
+                   const std::vector<double> &defocus, const CTF &c,
+                   double pixel_size, float *out, eDevice device,
+                   int gpu_index) {
+  if (device != e_device) host_device_unsupported();
+  gx_stack_desc d{};
+  d.num_pixels = xsize;
+  d.num_rows = ysize;
+  d.num_images = num_images;
+  d.num_defocus = defocus.size();
+  d.defocus = defocus.data();
+  d.pixel_size = pixel_size;
+  d.wavelength = c.l;
+  d.Cs = c.Cs;
+  d.Ca = c.Ca;
+  d.Pa = c.Pa;
+  d.phi = c.phi;
+  d.gpu_index = gpu_index;
+  check_status(gx_correct_stack(&d, images, out));
+}
+
 // ---- CTF physics (ctf.h), FP64 ----------------------------------------------
 
 namespace {

@@ -81,6 +81,16 @@ void correct(const float *image, const std::complex<float> *ctf, float *rec,
              std::size_t xsize, std::size_t ysize, std::size_t num_ctf,
              eDevice device, int gpu_index = -1);
 
+// A stack of images (num_images x ysize x xsize) phase flipped for every
+// defocus into out (num_images x defocus.size() x ysize x xsize), the CTF
+// evaluated on the device. c.df is not read.
+struct CTF;
+void correct_stack(const float *images, std::size_t num_images,
+                   std::size_t xsize, std::size_t ysize,
+                   const std::vector<double> &defocus, const CTF &c,
+                   double pixel_size, float *out, eDevice device,
+                   int gpu_index = -1);
+
 // ---- CTF physics, FP64 (ctf.h) ---------------------------------------------
 
 // ctf.h:167-178

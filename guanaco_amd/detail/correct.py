@@ -132,14 +132,26 @@ def correct_projections(projections, centre=None, pixel_size=1, energy=None,
     assert abs(mn + (ndf - 1) * step - mx) < 1e-7, "Inconsistent defocus steps"
     T, Y, X = projections.shape
     corrected = get_corrected_array((T, ndf, Y, X), corrected_output)
-    ctf = get_ctf_array(X, Y, pixel_size, energy, mn, ndf, step,
-                        spherical_aberration, astigmatism, astigmatism_angle,
-                        phase_shift)
-    buf = numpy.empty((ndf, Y, X), numpy.float32)
-    for z in range(T):
-        image = numpy.ascontiguousarray(projections[z], dtype=numpy.float32)
-        ext.corr(image, ctf, buf, device)
-        corrected[z] = buf
+    # the CTF of get_ctf() without its defocus: the device evaluates it for
+    # every slab, in the same FP64 arithmetic
+    ctf = ext.CTF(l=ext.get_electron_wavelength(energy * 1000),
+                  Cs=spherical_aberration * 1e7, Ca=astigmatism,
+                  Pa=astigmatism_angle * pi / 180, phi=phase_shift * pi / 180)
+    defoci = [float(mn + d * step) for d in range(ndf)]
+    # blocks of tilts of about 256 MiB of results, written in place where the
+    # output is plain float32 memory
+    n = max(1, (256 << 20) // (4 * ndf * Y * X))
+    direct = (isinstance(corrected, numpy.ndarray)
+              and corrected.dtype == numpy.float32
+              and corrected.flags.c_contiguous and corrected.flags.writeable)
+    for z in range(0, T, n):
+        images = numpy.ascontiguousarray(projections[z:z + n],
+                                         dtype=numpy.float32)
+        out = numpy.asarray(corrected[z:z + n]) if direct else numpy.empty(
+            (images.shape[0], ndf, Y, X), numpy.float32)
+        ext.correct_stack(images, out, defoci, ctf, pixel_size, device)
+        if not direct:
+            corrected[z:z + n] = out
     if ndf == 1:
         corrected = corrected.reshape(projections.shape)
     return corrected, mn - defocus, mx - defocus

@@ -136,6 +136,28 @@ int gx_filter(const float *rows, float *out, size_t nrows, size_t num_pixels,
 int gx_corr(const float *image, const float *ctf, float *rec, size_t xsize,
             size_t ysize, size_t num_ctf, int gpu_index);
 
+/* No counterpart in the reference: gx_corr of a stack of images with the CTFs
+ * of one microscope, which the device evaluates itself (as the volume path
+ * does), so that neither the CTF images nor their uploads are needed. images
+ * (num_images x num_rows x num_pixels, host), out (num_images x num_defocus x
+ * num_rows x num_pixels, host, overwritten): out[i][k] is image i phase
+ * flipped with the absolute defocus defocus[k], as correct_projections does
+ * (correct.py:217-318). Several images per launch and per copy. Sizes as
+ * gx_corr. Synchronous. */
+typedef struct gx_stack_desc {
+  size_t num_pixels, num_rows, num_images, num_defocus;
+  const double *defocus; /* host, num_defocus, A */
+  double pixel_size;     /* A */
+  double wavelength;     /* A */
+  double Cs;             /* A */
+  double Ca;             /* A */
+  double Pa;             /* rad */
+  double phi;            /* rad */
+  int gpu_index;         /* -1 = current device */
+} gx_stack_desc;
+int gx_correct_stack(const gx_stack_desc *desc, const float *images,
+                     float *out);
+
 /* CTF images on the FFT-ordered grid, computed on the device in FP64 and
  * stored as complex64: out[k][y][x] (interleaved re, im) for the absolute
  * defocus defocus[k]. With envelope, CTF.get_ctf(w, h, ps) of the reference
