@@ -20,10 +20,9 @@
 // kBF16 (whose error budget is set by the storage) compute p with two fused
 // multiply-adds from a table holding offset - 1/2 and the scale times the
 // normalisation the filter pass divided out, and accumulate with FP32 fused
-// multiply-adds (BF16 taps rounded to FP16 first: bf16_tap); here they have
-// the direct kernels only (narrow slabs, one centre per row), the other
-// plans run on the matrix cores (gx_bp_mm.hip). The per-tilt tables are read
-// with scalar loads.
+// multiply-adds (BF16 taps rounded to FP16 first: bf16_tap). The per-tilt
+// tables are read with scalar loads. 16-bit plans with one slab, and large
+// ones with wide slabs, run on the matrix cores instead (gx_bp_mm.hip).
 #include <type_traits>
 
 #include "gx_bp_geometry.hpp"
@@ -37,13 +36,22 @@ constexpr int kTX = 32, kTZ = 8;
 template <int YB, int STORE>
 struct Taps;
 
-// BF16 taps enter the arithmetic rounded to FP16, as the matrix-core kernel
-// keeps them in LDS: exact for magnitudes in [2^-14, 65504] (eight
-// significant bits fit FP16's eleven), and within 2^-25 below, where FP16 is
-// subnormal. The normalised slabs stay far below 65504, as they must for FP16
-// storage.
+// BF16 taps enter the arithmetic rounded to FP16, as the staged kernel keeps
+// them in LDS (bf16_pair_to_f16): exact for magnitudes in [2^-14, 65504]
+// (eight significant bits fit FP16's eleven), and within 2^-25 below, where
+// FP16 is subnormal. The normalised slabs stay far below 65504, as they must
+// for FP16 storage. The staged kernel then interpolates with
+// v_fma_mix_f32, one instruction per tap, like FP16, where BF16 would need a
+// shift or mask before each FMA; the direct kernels round the same way so
+// that every kernel gives the same bits.
 __device__ __forceinline__ float bf16_tap(float v) {
   return (float)(_Float16)v;
+}
+__device__ __forceinline__ uint32_t bf16_pair_to_f16(uint32_t w) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  const f32x2 f = {__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u)};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
 }
 template <int STORE>
 __device__ __forceinline__ float tap_value(typename StoreT<STORE>::T v) {
@@ -116,6 +124,13 @@ struct Taps {
 #pragma unroll
     for (int i = 0; i < YB / 8; ++i) unpack(i, q0[i], q1[i]);
   }
+  // The staged kernel's word-major runs: word i of position p at q[i SW]
+  // (q at position p), position p + 1 one word on.
+  template <int SW>
+  __device__ __forceinline__ void load16_strided(const uint4 *q) {
+#pragma unroll
+    for (int i = 0; i < YB / 8; ++i) unpack(i, q[i * SW], q[i * SW + 1]);
+  }
   __device__ __forceinline__ static float lo(uint32_t w) {
     if constexpr (STORE == kF16) {
       return __half2float(__ushort_as_half((unsigned short)(w & 0xffffu)));
@@ -177,7 +192,7 @@ hipError_t launch_bp_coefficients(const float4 *coef, const uint32_t *tmax,
 }
 
 // ---------------------------------------------------------------------------
-// LDS-staged form (float32 slabs).
+// LDS-staged form.
 //
 // p is a chain of correctly rounded float operations, each monotone in x and
 // in z, so over a 32 x 8 tile i0 is smallest at one of the four corners, and
@@ -197,13 +212,15 @@ hipError_t launch_bp_coefficients(const float4 *coef, const uint32_t *tmax,
 // values, never an access outside the buffer.
 //
 // The runs are loaded straight into LDS (buffer_load ... lds), not through
-// registers. Two LDS buffers: the loads of batch b + 1 are issued before
-// batch b is interpolated, one barrier per batch. FP32 slabs only.
+// registers; BF16 runs are then converted to FP16 in place by the lanes that
+// loaded them (bf16_tap). Two LDS buffers: the loads of batch b + 1 are
+// issued before batch b is interpolated, one barrier per batch.
 constexpr int kWPOS = 40;
 
-template <int YB, int KS>
+template <int YB, int STORE, int KS>
 struct Staging {
-  static constexpr int kPosBytes = YB * (int)sizeof(float);
+  using T = typename StoreT<STORE>::T;
+  static constexpr int kPosBytes = YB * (int)sizeof(T);
   static constexpr int kPosWords = kPosBytes / 16;      // 16-byte words
   static constexpr int kTB = 256 / (kPosBytes * KS);    // tilts per batch
   static constexpr int kNSlot = kTB * KS;  // (tilt, slab) runs per batch
@@ -230,7 +247,7 @@ struct Staging {
 constexpr int kOneSlab = 1 << 30;
 constexpr int kSlabMask = kOneSlab - 1;
 
-template <bool MULTI>
+template <bool EXACT, bool MULTI>
 __device__ __forceinline__ int2 tile_window(float4 cf, float x0, float x1,
                                             float z0, float z1, float dscale,
                                             float doffset, int ndf) {
@@ -240,7 +257,7 @@ __device__ __forceinline__ int2 tile_window(float4 cf, float x0, float x1,
     const float x = (c & 1) ? x1 : x0;
     const float z = (c & 2) ? z1 : z0;
     float tt;
-    w = min(w, tap_index<true>(x, z, cf, tt));
+    w = min(w, tap_index<EXACT>(x, z, cf, tt));
     if constexpr (MULTI) {
       const int kc = slab_of(x, z, cf, dscale, doffset, ndf);
       k = min(k, kc);
@@ -251,7 +268,7 @@ __device__ __forceinline__ int2 tile_window(float4 cf, float x0, float x1,
 }
 
 // win[tile * Tpad + t], tile = bx * nbz + bz (the kernels' order).
-template <bool MULTI>
+template <bool EXACT, bool MULTI>
 __global__ void k_bp_windows(const float4 *__restrict__ coef, int T, int Tpad,
                              int W, int Z, int nbx, int nbz, float dscale,
                              float doffset, int ndf, int2 *__restrict__ win) {
@@ -266,7 +283,8 @@ __global__ void k_bp_windows(const float4 *__restrict__ coef, int T, int Tpad,
     const float x1 = voxel_coord(min(bx * kTX + kTX, W) - 1, W);
     const float z0 = voxel_coord(bz * kTZ, Z);
     const float z1 = voxel_coord(min(bz * kTZ + kTZ, Z) - 1, Z);
-    r = tile_window<MULTI>(coef[t], x0, x1, z0, z1, dscale, doffset, ndf);
+    r = tile_window<EXACT, MULTI>(coef[t], x0, x1, z0, z1, dscale, doffset,
+                                  ndf);
   }
   win[i] = r;
 }
@@ -276,19 +294,26 @@ size_t bp_window_entries(int W, int Z, int T) {
   return nbx * nbz * (size_t)bp_tilt_pad(T);
 }
 
-hipError_t launch_bp_windows(const float4 *coef, int T, int W, int Z,
-                             float dscale, float doffset, int ndf, int2 *win,
-                             hipStream_t s) {
+hipError_t launch_bp_windows(const float4 *coef, int exact, int T, int W,
+                             int Z, float dscale, float doffset, int ndf,
+                             int2 *win, hipStream_t s) {
   const int nbx = (W + kTX - 1) / kTX, nbz = (Z + kTZ - 1) / kTZ;
   const size_t n = bp_window_entries(W, Z, T);
   const dim3 g((unsigned)((n + 255) / 256)), b(256);
   const int Tpad = bp_tilt_pad(T);
-  if (ndf > 1)
-    hipLaunchKernelGGL(k_bp_windows<true>, g, b, 0, s, coef, T, Tpad, W, Z,
-                       nbx, nbz, dscale, doffset, ndf, win);
+  const bool multi = ndf > 1;
+  if (exact && multi)
+    hipLaunchKernelGGL((k_bp_windows<true, true>), g, b, 0, s, coef, T, Tpad,
+                       W, Z, nbx, nbz, dscale, doffset, ndf, win);
+  else if (exact)
+    hipLaunchKernelGGL((k_bp_windows<true, false>), g, b, 0, s, coef, T, Tpad,
+                       W, Z, nbx, nbz, dscale, doffset, ndf, win);
+  else if (multi)
+    hipLaunchKernelGGL((k_bp_windows<false, true>), g, b, 0, s, coef, T, Tpad,
+                       W, Z, nbx, nbz, dscale, doffset, ndf, win);
   else
-    hipLaunchKernelGGL(k_bp_windows<false>, g, b, 0, s, coef, T, Tpad, W, Z,
-                       nbx, nbz, dscale, doffset, ndf, win);
+    hipLaunchKernelGGL((k_bp_windows<false, false>), g, b, 0, s, coef, T, Tpad,
+                       W, Z, nbx, nbz, dscale, doffset, ndf, win);
   return hipGetLastError();
 }
 
@@ -516,16 +541,19 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_rows(
   }
 }
 
-template <int YB, bool MULTI, int KS>
+template <int YB, int STORE, bool MULTI, int KS>
 __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
-    const float *__restrict__ slab,
+    const typename StoreT<STORE>::T *__restrict__ slab,
     const float4 *__restrict__ coef, const int2 *__restrict__ win,
     float dscale, float doffset, int ndf, int N, int T, int NYB, int W, int Z,
     int Y, int yb0, int y_base, int slab_yb0, float *__restrict__ vol,
     int nbx, int nbz,
     unsigned nblocks) {
-  using S = Staging<YB, KS>;
-  using ST = float;
+  using S = Staging<YB, STORE, KS>;
+  using ST = typename StoreT<STORE>::T;
+  constexpr bool kExact = STORE == kF32;
+  // BF16 runs are staged as FP16 (bf16_tap)
+  constexpr int kLds = STORE == kBF16 ? kF16 : STORE;
   static_assert(MULTI || KS == 1, "one slab without defocus slabs");
   // Two buffers as two arrays: with distinct objects the compiler can tell
   // that reads of one do not wait for the direct loads into the other.
@@ -591,6 +619,24 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
                       dslot[c] >= 0 ? base + dslot[c] : -1);
     }
   };
+  // After this wave's loads have landed: BF16 slots to FP16, each by the
+  // lane that loaded it (no other wave touches them before the barrier).
+  auto convert_batch = [&](uint4 *dst) {
+    if constexpr (STORE == kBF16) {
+#pragma unroll
+      for (int i = 0; i < S::kSPW; ++i) {
+        const int q = wave + (kTX * kTZ / 64) * i;
+#pragma unroll
+        for (int c = 0; c < S::kCPL; ++c) {
+          uint4 *d = dst + q * S::kRunSlots + lane + 64 * c;
+          const uint4 v = *d;
+          *d = make_uint4(bf16_pair_to_f16(v.x), bf16_pair_to_f16(v.y),
+                          bf16_pair_to_f16(v.z), bf16_pair_to_f16(v.w));
+        }
+      }
+    }
+  };
+
   float acc[YB];
 #pragma unroll
   for (int r = 0; r < YB; ++r) acc[r] = 0.0f;
@@ -626,14 +672,14 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
           }
         }
         float tt;
-        const int i0 = tap_index<true>(x, z, cf, tt);
+        const int i0 = tap_index<kExact>(x, z, cf, tt);
         if (active && (unsigned)i0 < (unsigned)(N - 1)) {
           const int rel = min(max(i0 - w.x, 0), kWPOS - 2);
           // word-major run: word wi of position p in slot wi kWPOS + p
-          Taps<YB, kF32> tp;
+          Taps<YB, kLds> tp;
           tp.template load16_strided<kWPOS>(cur + (j * KS + ks) * S::kRunSlots +
                                             rel);
-          accumulate<YB, kF32>(acc, tp, cf, tt);
+          accumulate<YB, kLds>(acc, tp, cf, tt);
         }
       }
     }
@@ -641,12 +687,14 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
       // this wave's loads have landed; the barrier then covers the other
       // waves' too
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      convert_batch(nxt);
     }
     lds_barrier();
   };
 
   load_batch(0, lds_a);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  convert_batch(lds_a);
   lds_barrier();
   const int nb = (T + S::kTB - 1) / S::kTB;
   for (int b = 0; b < nb; b += 2) {
@@ -663,27 +711,28 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_lds(
 }
 
 // ------------------------------------------------------------ launchers ---
-template <int YB, bool MULTI, int KS>
+template <int YB, int STORE, bool MULTI, int KS>
 static hipError_t launch_bp_lds_k(const BpArgs &a, hipStream_t s) {
+  using ST = typename StoreT<STORE>::T;
   const int nbx = (a.W + kTX - 1) / kTX;
   const int nbz = (a.Z + kTZ - 1) / kTZ;
   if (a.yb1 <= a.yb0) return hipSuccess;
   if (a.win == nullptr) return hipErrorInvalidValue;
   const unsigned nb =
       (unsigned)nbx * (unsigned)nbz * (unsigned)(a.yb1 - a.yb0);
-  hipLaunchKernelGGL((k_bp_lds<YB, MULTI, KS>), dim3(nb), dim3(kTX * kTZ), 0,
-                     s, (const float *)a.slab, a.coef, a.win, a.dscale,
-                     a.doffset, a.ndf, a.N, a.T, a.NYB, a.W, a.Z, a.Y, a.yb0,
-                     a.y_base, a.slab_yb0, a.vol, nbx, nbz, nb);
+  hipLaunchKernelGGL((k_bp_lds<YB, STORE, MULTI, KS>), dim3(nb),
+                     dim3(kTX * kTZ), 0, s, (const ST *)a.slab, a.coef, a.win,
+                     a.dscale, a.doffset, a.ndf, a.N, a.T, a.NYB, a.W, a.Z,
+                     a.Y, a.yb0, a.y_base, a.slab_yb0, a.vol, nbx, nbz, nb);
   return hipGetLastError();
 }
 
-template <int YB>
+template <int YB, int STORE>
 static hipError_t launch_bp_lds_t(const BpArgs &a, hipStream_t s) {
-  if (a.ndf == 1) return launch_bp_lds_k<YB, false, 1>(a, s);
+  if (a.ndf == 1) return launch_bp_lds_k<YB, STORE, false, 1>(a, s);
   switch (a.staged) {
-    case 2: return launch_bp_lds_k<YB, true, 2>(a, s);
-    case 4: return launch_bp_lds_k<YB, true, 4>(a, s);
+    case 2: return launch_bp_lds_k<YB, STORE, true, 2>(a, s);
+    case 4: return launch_bp_lds_k<YB, STORE, true, 4>(a, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -750,8 +799,16 @@ hipError_t launch_bp(const BpArgs &a, int YB, int store, hipStream_t s) {
     return hipErrorInvalidValue;
   }
   if (a.staged) {
-    if (store == kF32 && YB == 8) return launch_bp_lds_t<8>(a, s);
-    if (store == kF32 && YB == 16) return launch_bp_lds_t<16>(a, s);
+    if (store == kF32) {
+      if (YB == 8) return launch_bp_lds_t<8, kF32>(a, s);
+      if (YB == 16) return launch_bp_lds_t<16, kF32>(a, s);
+    } else if (store == kF16) {
+      if (YB == 16) return launch_bp_lds_t<16, kF16>(a, s);
+      if (YB == 32) return launch_bp_lds_t<32, kF16>(a, s);
+    } else if (store == kBF16) {
+      if (YB == 16) return launch_bp_lds_t<16, kBF16>(a, s);
+      if (YB == 32) return launch_bp_lds_t<32, kBF16>(a, s);
+    }
     return hipErrorInvalidValue;
   }
   if (store == kF32) {

@@ -66,6 +66,7 @@ constexpr int kPos = 24;     // staged positions
 constexpr int kMaxBase = kPos - 8;
 constexpr int kExtra = 2;    // runs of second and third slabs per batch
 constexpr int kWaves = 8;
+constexpr size_t kFill = 256;
 // window table: .y = first slab | (slabs - 1) << kSpanShift
 constexpr int kSpanShift = 28;
 constexpr int kSlabMask = (1 << kSpanShift) - 1;
@@ -331,6 +332,7 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
   const size_t tstride = (size_t)NYB * row_len;
   const uint16_t *rows = slab + (size_t)(byb - slab_yb0) * row_len;
   const int nyb = min(kYG, yb1 - byb);
+  const bool many = nyb * YB > 64;
   const int records = nyb * (int)row_len * 2;
   const int part = S::kSplit == 2 ? wave & 1 : 0;
   const int slot_w = wave / S::kSplit;  // the slot this wave loads
@@ -506,7 +508,8 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
           half8 bv[4];
           read_tr8x4<0, kBlock>(q, bv[0], bv[1], bv[2], bv[3]);
           tiles(Int<0>(), Int<4>(), bv);
-          if constexpr (RB == 4) {
+          // (a last workgroup with at most 64 rows left has no more)
+          if (RB == 4 && many) {
             read_tr8x4<2 * kBlock, kBlock>(q, bv[0], bv[1], bv[2], bv[3]);
             tiles(Int<4>(), Int<4>(), bv);
           }
@@ -653,22 +656,30 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
       *reinterpret_cast<float4v *>(q) = v * down;
     }
     lds_barrier();
+    if (wide) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = 2 * wave + i;
-      const int y = byb * YB + 16 * r + row;
-      const int oz = bz * kTile + (lane >> 2), ox = bx * kTile + 4 * (lane & 3);
-      const float4v v = *reinterpret_cast<const float4v *>(
-          out + row * S::kOutRow + 4 * lane);
-      if (y < Y && oz < Z && ox < W) {
-        float *d = vol + ((size_t)(y - y_base) * Z + oz) * W + ox;
-        if (wide) {
-          *reinterpret_cast<float4v *>(d) = v;
-        } else {
+      for (int i = 0; i < 2; ++i) {
+        const int row = 2 * wave + i;
+        const int y = byb * YB + 16 * r + row;
+        const int oz = bz * kTile + (lane >> 2);
+        const int ox = bx * kTile + 4 * (lane & 3);
+        if (y < Y && oz < Z && ox < W)
+          *reinterpret_cast<float4v *>(
+              vol + ((size_t)(y - y_base) * Z + oz) * W + ox) =
+              *reinterpret_cast<const float4v *>(out + row * S::kOutRow +
+                                                 4 * lane);
+      }
+    } else {
+      // lines of W values are not whole 16-byte words: a lane per voxel
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (ox + j < W) d[j] = v[j];
-        }
+      for (int i = 0; i < 8; ++i) {
+        const int row = 2 * wave + (i >> 2);
+        const int y = byb * YB + 16 * r + row;
+        const int oz = bz * kTile + 4 * (i & 3) + (lane >> 4);
+        const int ox = bx * kTile + (lane & 15);
+        if (y < Y && oz < Z && ox < W)
+          vol[((size_t)(y - y_base) * Z + oz) * W + ox] =
+              out[row * S::kOutRow + 64 * (i & 3) + lane];
       }
     }
   }
@@ -694,11 +705,35 @@ static hipError_t launch_mm(const BpArgs &a, hipStream_t s) {
 
 template <int YB, int STORE, bool MULTI>
 static hipError_t launch_mm_rows(const BpArgs &a, hipStream_t s) {
-  // rows per workgroup: 128, fewer where the volume has no more
+  // Rows per workgroup: 128, so that a block's weights serve as many rows as
+  // the registers hold; 64 or 32 where the volume has no more, or where
+  // larger workgroups would leave CUs without one (256 of them). The result
+  // does not depend on it.
   const int nrb = ((a.yb1 - a.yb0) * YB + 31) / 32;
-  if (nrb >= 3) return launch_mm<YB, STORE, MULTI, 4>(a, s);
-  if (nrb == 2) return launch_mm<YB, STORE, MULTI, 2>(a, s);
+  const size_t tiles = (size_t)((a.W + kTile - 1) / kTile) *
+                       ((a.Z + kTile - 1) / kTile);
+  if (nrb > 2 && tiles * ((nrb + 3) / 4) > kFill)
+    return launch_mm<YB, STORE, MULTI, 4>(a, s);
+  if (nrb > 1 && tiles * ((nrb + 1) / 2) > kFill)
+    return launch_mm<YB, STORE, MULTI, 2>(a, s);
   return launch_mm<YB, STORE, MULTI, 1>(a, s);
+}
+
+// With one slab always. With several, a workgroup's batches wait for window
+// entries and extra runs in turn, which takes other workgroups to hide and
+// wide slabs to be rare: two workgroups per CU (512) and slabs of at least 64
+// pixels. Measured against the staged kernel on the vector units, FP16, 61
+// tilts: 512 x 128 x 256 voxels (512 workgroups), slabs of 46, 64 and 102
+// pixels: 1.10, 1.12 and 1.33 times as fast; 640 x 150 x 200 (800), 53: 0.87;
+// 256 x 64 x 256 (128), 64: 0.72; 768 x 100 x 100 (336), 150: 0.77. Lines of
+// whole 16-byte words, as others cost it the rest (483 x 156 x 400, 161: the
+// request 0.99). Of the volume's rows, not of a band's: the kernels differ in
+// the last bit.
+bool bp_mm_suits(int ndf, float dscale, int W, int Z, int Y) {
+  if (ndf == 1) return true;
+  const size_t groups = (size_t)((W + kTile - 1) / kTile) *
+                        ((Z + kTile - 1) / kTile) * ((Y + 127) / 128);
+  return groups >= 512 && W % 4 == 0 && fabsf(dscale) * 64.0f <= 1.0f;
 }
 
 hipError_t launch_bp_mm(const BpArgs &a, int YB, int store, hipStream_t s) {

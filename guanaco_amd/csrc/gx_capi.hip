@@ -852,8 +852,7 @@ struct gx_volume_plan {
   int band = 0, slab_y0 = 0, slab_y1 = 0;
   int bp_kind = GX_BP_STAGED;
   int bp_staged = 1;  // slabs per tilt of the staged kernel; 0 = direct
-  // 16-bit slabs of a plan with one centre whose tiles span at most
-  // bp_staged slabs: both kinds run the matrix-core kernel
+  // 16-bit slabs on the matrix cores, whatever bp_kind (plan_mm)
   bool bp_mm = false;
   bool ctf = false;
   float dscale = 0, doffset = 0, nrm_mul = 1;
@@ -985,7 +984,9 @@ bool plan_mm(const gx_volume_desc *d) {
   defocus_coefficients(d->num_defocus, d->pixel_size, d->min_defocus,
                        d->max_defocus, &dscale, &doffset);
   return d->storage != GX_STORE_F32 && d->centres == nullptr &&
-         bp_slots(d->num_defocus, dscale) != 0;
+         bp_slots(d->num_defocus, dscale) != 0 &&
+         bp_mm_suits((int)d->num_defocus, dscale, (int)d->width,
+                     (int)d->depth, (int)d->num_rows);
 }
 size_t plan_windows(int W, int Z, int T, bool mm) {
   return mm ? bp_mm_window_entries(W, Z, T) : bp_window_entries(W, Z, T);
@@ -1200,7 +1201,7 @@ int plan_upload(gx_volume_plan *p, hipStream_t s) {
                         hipMemcpyHostToDevice, s));
   // the staged kernel's windows, with the arithmetic of the plan's kernels
   if (p->storage == GX_STORE_F32) {
-    GX_HIP(launch_bp_windows(p->coef.as<float4>(), p->T, p->W, p->Z,
+    GX_HIP(launch_bp_windows(p->coef.as<float4>(), 1, p->T, p->W, p->Z,
                              p->dscale, p->doffset, p->ndf, p->win.as<int2>(),
                              s));
   } else {
@@ -1210,8 +1211,8 @@ int plan_upload(gx_volume_plan *p, hipStream_t s) {
       GX_HIP(launch_bp_mm_windows(p->coef_r.as<float4>(), p->T, p->W, p->Z,
                                   p->dscale, p->doffset, p->ndf,
                                   p->win.as<int2>(), s));
-    else if (p->per_row)  // (its slabs only: the same in every storage)
-      GX_HIP(launch_bp_windows(p->coef.as<float4>(), p->T, p->W, p->Z,
+    else
+      GX_HIP(launch_bp_windows(p->coef_r.as<float4>(), 0, p->T, p->W, p->Z,
                                p->dscale, p->doffset, p->ndf,
                                p->win.as<int2>(), s));
   }

@@ -148,16 +148,17 @@ hipError_t launch_bp(const BpArgs &a, int YB, int store, hipStream_t s);
 hipError_t launch_bp_coefficients(const float4 *coef, const uint32_t *tmax,
                                   float nrm_mul, int T, float4 *out,
                                   hipStream_t s);
-// Window table of the staged kernel (float32 slabs): bp_window_entries(W, Z,
-// T) int2, from the reference's coefficients.
+// Window table of the staged kernel: bp_window_entries(W, Z, T) int2, from
+// the coefficient table the kernels read (exact != 0: kF32 arithmetic).
 size_t bp_window_entries(int W, int Z, int T);
-hipError_t launch_bp_windows(const float4 *coef, int T, int W, int Z,
-                             float dscale, float doffset, int ndf,
+hipError_t launch_bp_windows(const float4 *coef, int exact, int T, int W,
+                             int Z, float dscale, float doffset, int ndf,
                              int2 *win, hipStream_t s);
 
-// The matrix-core kernel of 16-bit slabs (one centre, a tile spans at most
-// four slabs; a.win from launch_bp_mm_windows): any rows per block YB that
-// the storage has.
+// The matrix-core kernel of 16-bit slabs (one centre, a 16 x 16 tile spans at
+// most three slabs; a.win from launch_bp_mm_windows): any rows per block YB
+// that the storage has. bp_mm_suits: the plans it is the faster kernel for.
+bool bp_mm_suits(int ndf, float dscale, int W, int Z, int Y);
 hipError_t launch_bp_mm(const BpArgs &a, int YB, int store, hipStream_t s);
 // Its window table, bp_mm_window_entries(W, Z, T) int2.
 size_t bp_mm_window_entries(int W, int Z, int T);

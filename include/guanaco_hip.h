@@ -271,10 +271,10 @@ int gx_volume_rows_per_block(gx_volume_plan *plan, size_t *rows);
  * copies each voxel tile's detector window into LDS per batch of tilts and
  * holds 1, 2 or 4 defocus slabs per tilt; when a tile spans more slabs
  * (narrow slabs, large |dscale|) plans use GX_BP_DIRECT, which gathers taps
- * straight from global memory. Both give identical results. With 16-bit
- * storage both names stand for the matrix-core kernel wherever the staged one
- * could run; the direct kernel remains for narrow slabs and for one rotation
- * centre per row. */
+ * straight from global memory. Both give identical results. For plans
+ * with 16-bit storage that run on the matrix cores (one slab, or several
+ * wide ones over a volume large enough to fill the GPU) both names stand for
+ * that one kernel. */
 #define GX_BP_DIRECT 0
 #define GX_BP_STAGED 1
 int gx_volume_plan_set_backprojector(gx_volume_plan *plan, int kind);
@@ -298,8 +298,8 @@ int gx_volume_plan_slab_range(gx_volume_plan *plan, int *first, int *last);
  * per thread; `rows` is also the row blocking of the filtered slabs. The
  * candidates are rows 8 and 16 for float32 slabs, 16 and 32 for float16 and
  * bfloat16 ones, each with the staged and the direct backprojector (staged
- * only where a tile spans at most 4 defocus slabs; one kernel, timed once,
- * stands for both with 16-bit slabs there). gx_volume_plan_autotune
+ * only where a tile spans at most 4 defocus slabs; timed once for both where
+ * the plan runs on the matrix cores). gx_volume_plan_autotune
  * filters d_in once per row count, times that filter pass and every
  * backprojector on the plan's own slabs with HIP events on `stream`, keeps
  * the candidate with the least filter + backprojection time, and leaves

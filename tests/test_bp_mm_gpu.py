@@ -2,11 +2,14 @@
 matrix-core kernel, and the kernel for one rotation centre per row.
 
 Each plan's own decoded slabs (times the per-tilt normalisation the filter
-divided out) are backprojected by the FP32 oracle. What is left is the FP32
-rounding of both sides and the weights' split into two FP16 parts: at most
-2^-22 per weight, and about (T + 8) 2^-24 of the sum of the terms'
-magnitudes in the accumulation, below 5e-6 for the 64 tilts used here at
-most; 1e-5 with the oracle's own rounding.
+divided out) are backprojected in FP64 with the taps and slabs that the
+storage's FP32 arithmetic gives (two fused multiply-adds for the position, as
+tests/test_bp_window.py emulates them; their rounding, an ulp of a position,
+is the storage's and not a kernel's). What is left is the FP32 rounding of
+the kernel and the weights' split into two FP16 parts: at most 2^-22 per
+weight, and about (T + 8) 2^-24 of the sum of the terms' magnitudes in the
+accumulation, below 5e-6 for the 64 tilts used here at most; 1e-5 with room
+for cancellation in the sums.
 """
 import numpy
 import pytest
@@ -28,12 +31,49 @@ CASES = [
     (48, 129, 5, 1, 33, 50, 80.0, (0.0, 0.0), None),
     # every quadrant, a detector narrower than a staged run
     (20, 65, 64, 1, 40, 36, 175.0, (0.0, 0.0), None),
-    # two and three slabs in a tile: extra runs, batches that close early
+    # several slabs, small: the staged kernel
     (96, 40, 21, 6, 50, 96, 65.0, (-100.0, 100.0), None),
     (80, 97, 30, 4, 80, 80, 70.0, (-25.0, 25.0), None),
+    # several wide slabs over a large volume: extra runs, batches that close
+    # early, a last workgroup with one row block; partial tiles
+    (260, 385, 9, 4, 130, 260, 70.0, (-130.0, 130.0), None),
+    (200, 450, 6, 3, 131, 268, 85.0, (-100.0, 100.0), None),
     # tilts of very different weight
     (64, 34, 12, 2, 20, 64, 60.0, (-90.0, 90.0), 1e-3),
 ]
+
+
+f32 = numpy.float32
+
+
+def fma32(a, b, c):
+    return (numpy.asarray(a, numpy.float64) * numpy.asarray(b, numpy.float64)
+            + numpy.asarray(c, numpy.float64)).astype(f32)
+
+
+def backproject(slabs, Z, W, angles, centre, mn, mx):
+    """(ndf, T, X) slab rows to a (Z, W) slice, FP64 sums of FP32 decisions
+    (1 pixel is 1 A)."""
+    ndf, T, X = slabs.shape
+    x = (numpy.arange(W) - 0.5 * W + 0.5).astype(f32)[None, :]
+    z = (numpy.arange(Z) - 0.5 * Z + 0.5).astype(f32)[:, None]
+    out = numpy.zeros((Z, W))
+    ds = f32(f32(ndf) / (f32(mx) - f32(mn))) if ndf > 1 else f32(0)
+    do = f32(-ds * f32(mn))
+    for t, (c, s, off, scale) in enumerate(O.tilt_coefficients(angles,
+                                                               centre)):
+        p = fma32(x, c, fma32(-z, s, f32(off) - f32(0.5)))
+        i = numpy.floor(p).astype(numpy.int64)
+        w = p.astype(numpy.float64) - i
+        d = (-x * f32(s) - z * f32(c)) * ds + do
+        k = numpy.clip(numpy.floor(d.astype(numpy.float64) + 0.5), 0,
+                       ndf - 1).astype(numpy.int64)
+        ok = (i >= 0) & (i < X - 1)
+        i = numpy.clip(i, 0, max(X - 2, 0))
+        r = slabs[:, t].astype(numpy.float64)
+        v = (1 - w) * r[k, i] + w * r[k, numpy.minimum(i + 1, X - 1)]
+        out += numpy.where(ok, float(scale) * v, 0.0)
+    return out
 
 
 def plan_of(case, storage):
@@ -92,15 +132,14 @@ def test_matches_oracle_on_its_own_slabs(capi, case, storage, rows):
     for t in range(T):  # slabs no voxel reads hold anything
         slabs[:first[t], t] = slabs[last[t] + 1:, t] = 0
     for y in sorted({0, Y // 3, Y // 2, Y - 1}):
-        s = numpy.ascontiguousarray(slabs[:, :, y])
-        expect = O.project(s if ndf > 1 else s[0], (Z, W), angles,
-                           X / 2.0 - 0.3, 1.0, mn, mx)
+        expect = backproject(slabs[:, :, y], Z, W, angles, X / 2.0 - 0.3, mn,
+                             mx)
         err = numpy.linalg.norm(vol[y] - expect)
         assert err <= 1e-5 * numpy.linalg.norm(expect), (y, err)
     plan.destroy()
 
 
-@pytest.mark.parametrize("case", [CASES[1], CASES[4], CASES[6]])
+@pytest.mark.parametrize("case", [CASES[1], CASES[4], CASES[6], CASES[7]])
 def test_exceptional_values_reach_only_their_voxels(capi, case):
     # A NaN in one row of one tilt makes that filtered row NaN, and the row
     # it is transformed with (rows 2i and 2i + 1 travel as one complex row):
@@ -169,8 +208,7 @@ def test_centre_per_row_matches_oracle_on_its_own_slabs(capi, case, storage,
         slabs[:first[t], t] = slabs[last[t] + 1:, t] = 0
     plan.destroy()
     for y in sorted({0, Y // 2, Y - 1}):
-        s = numpy.ascontiguousarray(slabs[:, :, y])
-        expect = O.project(s if ndf > 1 else s[0], (Z, W), angles,
-                           float(centres[y]), 1.0, mn, mx)
+        expect = backproject(slabs[:, :, y], Z, W, angles,
+                             float(centres[y]), mn, mx)
         err = numpy.linalg.norm(vol[y] - expect)
         assert err <= 1e-5 * numpy.linalg.norm(expect) + 1e-30, (y, err)
