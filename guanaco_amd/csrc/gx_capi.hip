@@ -173,32 +173,16 @@ int bp_slots(size_t ndf, float dscale) {
 // 1/(2N). L > 2N (N not a power of two): the reference's 2N-point filter as a
 // space kernel h (|d| <= N-1, all the zero-padded product can reach), then
 // its L-point DFT. Both give the reference's linear convolution.
-std::vector<float> ramp_table(size_t N, size_t L) {
-  std::vector<float> r(L / 2 + 1, 0.0f);
-  if (L == 2 * N) {
-    const float inv_l = 1.0f / (float)L;
-    for (size_t j = 0; j <= N; ++j) r[j] = ((float)j / (float)N) * inv_l;
-    return r;
-  }
-  const size_t M = 2 * N;
-  std::vector<double> cosM(M), cosL(L), h(N);
-  for (size_t i = 0; i < M; ++i) cosM[i] = std::cos(2.0 * M_PI * i / M);
-  for (size_t i = 0; i < L; ++i) cosL[i] = std::cos(2.0 * M_PI * i / L);
-  for (size_t d = 0; d < N; ++d) {
-    double acc = 0.0;
-    for (size_t k = 0; k < M; ++k) {
-      const size_t kk = k <= N ? k : M - k;
-      const double R = (double)((float)kk / (float)N);
-      acc += R * cosM[(k * d) % M];
-    }
-    h[d] = acc / (double)M;
-  }
-  for (size_t j = 0; j <= L / 2; ++j) {
-    double acc = h[0];
-    for (size_t d = 1; d < N; ++d) acc += 2.0 * h[d] * cosL[(j * d) % L];
-    r[j] = (float)(acc / (double)L);
-  }
-  return r;
+hipError_t make_ramp(size_t N, size_t L, float *d_ramp, double *scratch,
+                     std::vector<float> &host, hipStream_t s) {
+  if (L != 2 * N)
+    return launch_ramp_table((int)N, (int)L, scratch, d_ramp, s);
+  host.resize(N + 1);
+  const float inv_l = 1.0f / (float)L;
+  for (size_t j = 0; j <= N; ++j)
+    host[j] = ((float)j / (float)N) * inv_l;
+  return hipMemcpyAsync(d_ramp, host.data(), sizeof(float) * host.size(),
+                        hipMemcpyHostToDevice, s);
 }
 
 size_t filter_length(size_t N) {
@@ -212,7 +196,6 @@ namespace {
 
 using gx::defocus_coefficients;
 using gx::filter_length;
-using gx::ramp_table;
 using gx::tilt_geometry;
 
 // The power-of-two correction kernels take 8 <= X <= 8192 and 4 <= Y <=
@@ -601,15 +584,15 @@ static int filter_rows_dev(const float *d_in, float *d_out, size_t nrows,
                            size_t N, const float *d_wscale_ones,
                            hipStream_t s) {
   const size_t L = filter_length(N);
-  std::vector<float> r = ramp_table(N, L);
-  DevBuf d_ramp;
-  GX_HIP(d_ramp.alloc(sizeof(float) * r.size()));
-  GX_HIP(hipMemcpyAsync(d_ramp.p, r.data(), sizeof(float) * r.size(),
-                        hipMemcpyHostToDevice, s));
+  std::vector<float> r;
+  DevBuf d_ramp;  // the table's scratch, then the table
+  GX_HIP(d_ramp.alloc(sizeof(double) * N + sizeof(float) * (L / 2 + 1)));
+  float *ramp = (float *)(d_ramp.as<double>() + N);
+  GX_HIP(gx::make_ramp(N, L, ramp, d_ramp.as<double>(), r, s));
   // rows as (ndf = 1, T = nrows, Y = 1): slab layout [t][x] = input layout
   GX_HIP(launch_filter_rows(d_in, N, 0, 0, (int)N, (int)L, 1, (int)nrows, 1,
-                            d_ramp.as<float>(), d_wscale_ones, nullptr, 1.0f,
-                            kF32, d_out, 1, 1, s));
+                            ramp, d_wscale_ones, nullptr, 1.0f, kF32, d_out, 1,
+                            1, s));
   GX_HIP(hipStreamSynchronize(s));
   return GX_OK;
 }
@@ -1153,7 +1136,6 @@ void plan_setup(gx_volume_plan *p, const gx_volume_desc *d,
   p->h_wscale.assign(T, 1.0f);
   if (d->weights)
     for (size_t t = 0; t < T; ++t) p->h_wscale[t] = d->weights[t];
-  p->h_ramp = ramp_table(d->num_pixels, (size_t)ps.L);
   if (ps.ctf) p->h_defocus.assign(d->defocus, d->defocus + d->num_defocus);
   if (ps.ctf) {
     p->rows_bs = !rows_pow2(d->num_pixels);
@@ -1183,7 +1165,7 @@ void plan_buffers(gx_volume_plan *p, const PlanSizes &ps,
           sizeof(int2) * plan_windows(p->W, p->Z, p->T, p->bp_mm)},
          {&p->wscale, sizeof(float) * T},
          {&p->tmax, sizeof(uint32_t) * T},
-         {&p->ramp, sizeof(float) * p->h_ramp.size()},
+         {&p->ramp, sizeof(float) * ((size_t)ps.L / 2 + 1)},
          {&p->defocus, ps.ctf ? sizeof(double) * p->ndf : 0},
          {&p->mask, ps.mask_bytes},
          {&p->F, ps.f_bytes},
@@ -1235,9 +1217,10 @@ int plan_upload(gx_volume_plan *p, hipStream_t s) {
     GX_HIP(hipMemcpyAsync(p->row_off.p, p->h_row_off.data(),
                           sizeof(float) * p->h_row_off.size(),
                           hipMemcpyHostToDevice, s));
-  GX_HIP(hipMemcpyAsync(p->ramp.p, p->h_ramp.data(),
-                        sizeof(float) * p->h_ramp.size(),
-                        hipMemcpyHostToDevice, s));
+  // the slab buffer, which holds at least 64 bytes for each of the row's
+  // samples and nothing yet, is the table's scratch (8 bytes each)
+  GX_HIP(gx::make_ramp((size_t)p->X, (size_t)p->L, p->ramp.as<float>(),
+                       p->slab.as<double>(), p->h_ramp, s));
   // The slab buffer is not cleared: the filter writes every row below Y of
   // every slab the volume reads, and what else the backprojector reads (the
   // rows of the last row block past Y, the runs of slabs a tile does not use)

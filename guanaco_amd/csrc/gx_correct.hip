@@ -223,6 +223,59 @@ hipError_t launch_ctf_grid(float2 *out, int w, int h, double ps,
   return hipGetLastError();
 }
 
+// ----------------------------------------------------------- ramp table ---
+
+// The reference's 2N-point ramp (filter.cpp:30-45: float(k) / float(N)) as a
+// truncated space kernel and its L-point spectrum, for N that is no power of
+// two: sums of N cosines for each of N kernel values and L / 2 + 1 table
+// values, FP64, a wave each (fixed order). On the host these O(N^2) sums took
+// 9 ms at N = 1500, of each call that filters such rows; here about 20 us.
+__device__ __forceinline__ double wave_sum(double v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+
+// h[d] = (1 / 2N) sum_k R(k) cos(pi k d / N) over the symmetric 2N bins.
+__global__ __launch_bounds__(256) void k_ramp_kernel(int N,
+                                                     double *__restrict__ h) {
+  const int d = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (d >= N) return;
+  double acc = 0.0;
+  for (int k = (int)(threadIdx.x & 63); k <= N; k += 64) {
+    const double R = (double)((float)k / (float)N);
+    // k d mod 2N in integers, so that the argument is exact to rounding
+    const unsigned r = (unsigned)k * (unsigned)d % (2u * (unsigned)N);
+    const double c = R * cospi((double)r / (double)N);
+    acc += k == 0 || k == N ? c : 2.0 * c;
+  }
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) h[d] = acc / (2.0 * (double)N);
+}
+
+// out[j] = (1 / L) (h[0] + 2 sum_d h[d] cos(2 pi j d / L)), j <= L / 2.
+__global__ __launch_bounds__(256) void k_ramp_spectrum(
+    int N, int L, const double *__restrict__ h, float *__restrict__ out) {
+  const int j = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (j > L / 2) return;
+  double acc = 0.0;
+  for (int d = (int)(threadIdx.x & 63); d < N; d += 64) {
+    const unsigned r = (unsigned)j * (unsigned)d % (unsigned)L;
+    const double c = h[d] * cospi(2.0 * (double)r / (double)L);
+    acc += d == 0 ? c : 2.0 * c;
+  }
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) out[j] = (float)(acc / (double)L);
+}
+
+hipError_t launch_ramp_table(int N, int L, double *h, float *out,
+                             hipStream_t s) {
+  hipLaunchKernelGGL(k_ramp_kernel, dim3((unsigned)((N + 3) / 4)), dim3(256),
+                     0, s, N, h);
+  hipLaunchKernelGGL(k_ramp_spectrum, dim3((unsigned)((L / 2 + 1 + 3) / 4)),
+                     dim3(256), 0, s, N, L, h, out);
+  return hipGetLastError();
+}
+
 // ------------------------------------------------- pass 1: rows, R2C -------
 
 // 2 * RP image rows per workgroup (RP complex pairs). Writes the half

@@ -196,8 +196,14 @@ void slab_ranges(size_t T, const float *coef, int W, int Z, float dscale,
 void defocus_coefficients(size_t ndf, float ps, float mn, float mx,
                           float *dscale, float *doffset);
 // The reference's ramp filter (filter.cpp:30-45) for N samples on the
-// L-point grid, with the 1/L of the unnormalised inverse: L/2 + 1 values.
-std::vector<float> ramp_table(size_t N, size_t L);
+// L-point grid, with the 1/L of the unnormalised inverse: L/2 + 1 values at
+// d_ramp (device), in stream order. L = 2N: from `host`, which has to stay
+// until the copy is done. Else the 2N-point filter re-expressed on the device
+// (launch_ramp_table, scratch: N doubles of device memory).
+hipError_t make_ramp(size_t N, size_t L, float *d_ramp, double *scratch,
+                     std::vector<float> &host, hipStream_t s);
+hipError_t launch_ramp_table(int N, int L, double *h, float *out,
+                             hipStream_t s);
 // Filter transform length of N samples: a power of two >= 2N - 1, >= 8.
 size_t filter_length(size_t N);
 // Config checks of config.h:66-75 and the filter's size limit (GX_OK or a

@@ -3,8 +3,9 @@
 // For callers that cannot allocate device memory (code under graph capture,
 // tight serving loops, harnesses that forbid hipMalloc): the filtered copy
 // of the sinogram and the per-call tables live in `scratch`, a device global
-// of kScratchBytes, and the filter's twiddle factors in `noalloc_twiddles`,
-// another device global filled on the first call on a device. Every GPU the
+// of kScratchBytes, the filter's twiddle factors in `noalloc_twiddles`,
+// another device global filled on the first call on a device, and the sums
+// of the ramp table in `noalloc_ramp`. Every GPU the
 // library runs on holds its own copy of the arrays until the process ends,
 // and every call on that GPU shares them, so calls that overlap on one GPU
 // race. The kernels are gx_recon's.
@@ -24,12 +25,15 @@ using namespace gx;
 constexpr size_t kScratchBytes = (size_t)64 << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 static __device__ __align__(256) float2 noalloc_twiddles[tw_table_len()];
+// the ramp table's scratch (make_ramp): num_pixels doubles
+static __device__ __align__(256) double noalloc_ramp[8192];
 
 namespace {
 
 std::mutex g_mu;
 void *g_scratch[64] = {};   // per device: the address of its copy
 void *g_twiddles[64] = {};  // per device: its filled twiddle table
+void *g_ramp[64] = {};      // per device: noalloc_ramp
 
 int fail_hip(hipError_t e, const char *what) {
   char buf[256];
@@ -38,11 +42,11 @@ int fail_hip(hipError_t e, const char *what) {
   return fail_status(e == hipErrorOutOfMemory ? GX_ENOMEM : GX_EDEVICE, buf);
 }
 
-// This GPU's copies of `scratch` and `noalloc_twiddles`: the arrays' names
-// are host-side stand-ins, their device addresses come from
-// hipGetSymbolAddress, once per device with that device current; the
-// twiddle table is written then (a synchronous copy, no allocation).
-int device_arrays(void **scr, const float2 **tw) {
+// This GPU's copies of the arrays above: the names are host-side stand-ins,
+// their device addresses come from hipGetSymbolAddress, once per device with
+// that device current; the twiddle table is written then (a synchronous copy,
+// no allocation).
+int device_arrays(void **scr, const float2 **tw, double **ramp) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return fail_hip(e, "hipGetDevice");
@@ -50,13 +54,16 @@ int device_arrays(void **scr, const float2 **tw) {
     return fail_status(GX_EDEVICE, "gx_recon_noalloc: device index");
   std::lock_guard<std::mutex> lock(g_mu);
   if (g_scratch[dev] == nullptr) {
-    void *p = nullptr, *q = nullptr;
+    void *p = nullptr, *q = nullptr, *r = nullptr;
     e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
     if (e != hipSuccess) return fail_hip(e, "hipGetSymbolAddress(scratch)");
     e = hipGetSymbolAddress(&q, HIP_SYMBOL(noalloc_twiddles));
     if (e != hipSuccess)
       return fail_hip(e, "hipGetSymbolAddress(noalloc_twiddles)");
-    if (p == nullptr || q == nullptr)
+    e = hipGetSymbolAddress(&r, HIP_SYMBOL(noalloc_ramp));
+    if (e != hipSuccess)
+      return fail_hip(e, "hipGetSymbolAddress(noalloc_ramp)");
+    if (p == nullptr || q == nullptr || r == nullptr)
       return fail_status(GX_EDEVICE, "gx_recon_noalloc: no device address");
     const std::vector<float2> h = twiddle_host_table();
     e = hipMemcpy(q, h.data(), sizeof(float2) * h.size(),
@@ -64,7 +71,9 @@ int device_arrays(void **scr, const float2 **tw) {
     if (e != hipSuccess) return fail_hip(e, "twiddle table");
     g_scratch[dev] = p;
     g_twiddles[dev] = q;
+    g_ramp[dev] = r;
   }
+  *ramp = (double *)g_ramp[dev];
   *scr = g_scratch[dev];
   *tw = (const float2 *)g_twiddles[dev];
   return GX_OK;
@@ -106,7 +115,8 @@ extern "C" int gx_recon_noalloc(const gx_recon_cfg *cfg, const float *d_sino,
   if (cfg->gpu_index >= 0) NA_HIP(hipSetDevice(cfg->gpu_index));
   void *base = nullptr;
   const float2 *tw = nullptr;
-  rc = device_arrays(&base, &tw);
+  double *ramp_scratch = nullptr;
+  rc = device_arrays(&base, &tw, &ramp_scratch);
   if (rc) return rc;
   char *q = (char *)base;
   float *d_filt = (float *)q;
@@ -118,12 +128,11 @@ extern "C" int gx_recon_noalloc(const gx_recon_cfg *cfg, const float *d_sino,
   NA_HIP(hipStreamSynchronize(s));
   std::vector<float> coef(4 * T), ones(nrows, 1.0f);
   tilt_geometry(T, cfg->angles, cfg->centre, coef.data());
-  const std::vector<float> ramp = ramp_table(N, L);
+  std::vector<float> ramp;
   // synchronous copies: the host tables end with this call
   NA_HIP(hipMemcpy(d_coef, coef.data(), sizeof(float) * coef.size(),
                    hipMemcpyHostToDevice));
-  NA_HIP(hipMemcpy(d_ramp, ramp.data(), sizeof(float) * ramp.size(),
-                   hipMemcpyHostToDevice));
+  NA_HIP(make_ramp(N, L, d_ramp, ramp_scratch, ramp, s));
   NA_HIP(hipMemcpy(d_ones, ones.data(), sizeof(float) * nrows,
                    hipMemcpyHostToDevice));
   // reconstructor.cpp:92-115: filter a copy (the input is not modified),
