@@ -139,6 +139,20 @@ def test_matches_oracle_on_its_own_slabs(capi, case, storage, rows):
     plan.destroy()
 
 
+# depths about the tile order's limits: one strip of 16 tiles, then strips of
+# 8 with a last one of 1 (its one voxel deep), 2 and 8 tiles; two workgroups
+# of rows; several slabs
+@pytest.mark.parametrize("case", [
+    (60, 40, 5, 1, 256, 40, 60.0, (0.0, 0.0), None),
+    (60, 40, 5, 1, 257, 40, 60.0, (0.0, 0.0), None),
+    (60, 150, 5, 1, 277, 35, 80.0, (0.0, 0.0), None),
+    (60, 33, 5, 1, 384, 16, 60.0, (0.0, 0.0), None),
+    (300, 513, 5, 3, 281, 132, 70.0, (-180.0, 180.0), None),
+])
+def test_deep_volumes(capi, case):
+    test_matches_oracle_on_its_own_slabs(capi, case, "f16", 32)
+
+
 @pytest.mark.parametrize("case", [CASES[1], CASES[4], CASES[6], CASES[7]])
 def test_exceptional_values_reach_only_their_voxels(capi, case):
     # A NaN in one row of one tilt makes that filtered row NaN, and the row
