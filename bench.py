@@ -641,6 +641,12 @@ def load_counters(name):
     return out
 
 
+def bp_kernel(storage):
+    """The backprojection kernel of a workload's plans: the matrix-core
+    kernel for 16-bit slabs (every workload here is in its range)."""
+    return "k_bp_mm" if storage in ("f16", "bf16") else "k_bp_lds"
+
+
 def bp_roofline(w, entry, counters):
     """Roofline of the backprojection kernel of `entry`, timed live.
 
@@ -649,8 +655,10 @@ def bp_roofline(w, entry, counters):
     the FETCH_SIZE / WRITE_SIZE counters (committed summary of the same
     workload). What binds it is instruction issue: VALU instructions per
     SIMD per clock (counted instructions / this run's launch time) against
-    the FP32 issue rate probe kernels reach, and LDS bytes against the
-    measured ds_read_b128 peak. The gather model (two taps of s
+    the FP32 issue rate probe kernels reach (for the matrix-core kernel the
+    cycles its matrix and its other vector instructions take, since the two
+    hardly overlap), and LDS bytes against the measured ds_read_b128 peak.
+    The gather model (two taps of s
     bytes per update) is kept as a labelled figure: staging makes its taps
     LDS reads, so it exceeds the HBM peak."""
     X, Y, Z, T = w["X"], w["Y"], w["Z"], w["T"]
@@ -661,7 +669,8 @@ def bp_roofline(w, entry, counters):
     achieved = compulsory / (ms * 1e-3) / 1e9
     roof = {
         "bound": "hbm",
-        "kernel": "k_bp_lds (backprojection, %s slabs)" % entry["storage"],
+        "kernel": "%s (backprojection, %s slabs)" % (
+            bp_kernel(entry["storage"]), entry["storage"]),
         "achieved": achieved,
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
@@ -681,7 +690,19 @@ def bp_roofline(w, entry, counters):
         if traffic:
             roof["traffic_vs_algorithmic"] = traffic / compulsory
         simd_clk = NUM_CU * 4 * CLOCK_HZ * ms * 1e-3
-        if "valu_insts" in c:
+        if "mfma_insts" in c:
+            # SQ_INSTS_VALU counts the matrix instructions too
+            matrix = c["mfma_busy_cycles"] / simd_clk
+            vector = (c["valu_insts"] - c["mfma_insts"]) / (
+                VALU_ISSUE_PEAK * simd_clk)
+            roof["binding"] = {
+                "resource": "instruction issue (matrix + vector)",
+                "achieved": matrix + vector, "peak": 1.0,
+                "unit": "busy cycles per SIMD per clock",
+                "frac": matrix + vector, "matrix": matrix, "vector": vector,
+                "instructions_per_update": c["valu_insts"] * 64 / updates,
+            }
+        elif "valu_insts" in c:
             v = c["valu_insts"] / simd_clk
             roof["binding"] = {
                 "resource": "VALU issue",
@@ -846,7 +867,7 @@ def main():
                                        True)
     head = entry["paths"]["batched"]
     counters = load_counters("counters_%s_bp.txt" % args.config).get(
-        "k_bp_lds %s" % head["storage"], {})
+        "%s %s" % (bp_kernel(head["storage"]), head["storage"]), {})
     if counters:
         counters["_file"] = "counters_%s_bp.txt" % args.config
     line = {
