@@ -149,37 +149,50 @@ struct Taps {
 
 // ------------------------------------------------------- per-tilt tables --
 
-// out[t] = (c, s, offset - 1/2, scale * normalisation): the normalisation
-// float(tmax[t]) * nrm_mul is what the filter pass divided the stored values
-// by (1 where it is not positive, or without tmax). Entries T .. Tpad - 1 are
-// zero; entry Tpad holds (u, 1 / u): the power of two u that takes the
-// largest finite |scale| to [2^13, 2^14) (1 where there is none). One
-// workgroup.
+// out[t] = (c, s, offset - 1/2, weight): the weight is the tilt's scale times
+// the normalisation float(tmax[t]) * nrm_mul that the filter pass divided the
+// stored values by (1 without tmax), and zero for a tilt whose largest value
+// is zero: all it stored is zeros (or NaNs, which a zero weight keeps).
+// Entries T .. Tpad - 1 are zero. Entry Tpad is launch_bp_mm's: (u, 1 / u, 0),
+// the power of two u that takes the largest weight to [2^13, 2^14) (1 where
+// there is none). Its FP16 pairs end at 2^-24, which is finer than the FP32
+// rounding of a weight of at least 1; a series whose smallest weight falls
+// below that after scaling (tilts that differ 8192-fold), or with one that is
+// not finite, gets (1, 1, 1) and FP32 weights. One workgroup.
 __global__ __launch_bounds__(256) void k_bp_coefficients(
     const float4 *__restrict__ coef, const uint32_t *__restrict__ tmax,
     float nrm_mul, int T, int Tpad, float4 *__restrict__ out) {
   __shared__ float red[4];
-  float top = 0.0f;
+  float top = 0.0f, inv_low = 0.0f;  // (1 / the smallest, as a maximum)
   for (int t = threadIdx.x; t < Tpad; t += 256) {
     float4 r = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (t < T) {
       const float4 cf = coef[t];
-      float nrm = tmax != nullptr ? __uint_as_float(tmax[t]) * nrm_mul : 1.0f;
-      if (!(nrm > 0.0f)) nrm = 1.0f;
+      const float nrm =
+          tmax != nullptr ? __uint_as_float(tmax[t]) * nrm_mul : 1.0f;
       r = make_float4(cf.x, cf.y, cf.z - 0.5f, cf.w * nrm);
       const float a = fabsf(r.w);
-      if (a < __builtin_inff()) top = fmaxf(top, a);
+      if (!(a < __builtin_inff())) {
+        inv_low = __builtin_inff();
+      } else if (a > 0.0f) {
+        top = fmaxf(top, a);
+        inv_low = fmaxf(inv_low, 1.0f / a);
+      }
     }
     out[t] = r;
   }
   top = block_max<256>(top, red);
+  inv_low = block_max<256>(inv_low, red);
   if (threadIdx.x == 0) {
     int e = 0;
     if (top > 0.0f) {
       (void)frexpf(top, &e);  // top in [2^(e-1), 2^e)
       e = min(max(14 - e, -126), 126);
     }
-    out[Tpad] = make_float4(ldexpf(1.0f, e), ldexpf(1.0f, -e), 0.0f, 0.0f);
+    // smallest * u >= 1, also where 1 / smallest is infinite
+    const float u = ldexpf(1.0f, e);
+    out[Tpad] = inv_low <= u ? make_float4(u, ldexpf(1.0f, -e), 0.0f, 0.0f)
+                             : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
   }
 }
 

@@ -13,10 +13,12 @@
 // weights stay FP32 quantities: each is split into an FP16 high part and the
 // FP16 remainder (22 bits together), and both are multiplied, two matrix
 // instructions per product. The weights of all tilts are scaled by one power
-// of two that puts the largest in [2^13, 2^14), so that the remainders stay
-// normal FP16 numbers for tilts down to 2^-13 of it; the sum is scaled back
-// at the end. Detector position, tap and slab choice are the FP32 arithmetic
-// of the direct kernel.
+// of two that puts the largest in [2^13, 2^14), and the sum is scaled back at
+// the end. The pairs end at 2^-24: where a tilt's weight lies more than
+// 8192-fold below the largest, the series is computed tap by tap with FP32
+// weights instead (k_bp_coefficients decides; with one scale for every series
+// a 2^-40-fold weight was off by 8e-5 of its voxels). Detector position, tap
+// and slab choice are the FP32 arithmetic of the direct kernel.
 //
 // Work split. A workgroup is a 16 x 16 (x, z) tile by RB row blocks of 32
 // rows; each of its 8 waves holds two 4 x 4 blocks by all rows (64
@@ -349,6 +351,9 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
   const int2 *tw = win + (size_t)(bx * nbz + bz) * Tpad;
   const float up = kload(reinterpret_cast<const float *>(coef + Tpad), 0);
   const float down = kload(reinterpret_cast<const float *>(coef + Tpad), 1);
+  // weights too far apart for FP16 pairs (k_bp_coefficients): all tap by tap
+  const bool taps =
+      kload(reinterpret_cast<const float *>(coef + Tpad), 2) != 0.0f;
 
   // Staging: a lane's position and byte offset in a run, for the loads of
   // its wave (16-byte chunk c of the layout above).
@@ -563,7 +568,7 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int r = 0; r < kRT; ++r) acc[i][r] = (float4v)(0.0f);
-  {
+  if (!taps) {
     Batch b = next_batch(0);
     stage(b, lds);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -595,7 +600,7 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
     }
   }
 
-  bool bad = false;
+  bool bad = taps;
 #pragma unroll
   for (int r = 0; r < kRT; ++r) {
     const bool row = byb * YB + 16 * r + m < Y;
