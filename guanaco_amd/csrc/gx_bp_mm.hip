@@ -11,8 +11,14 @@
 // Precision. The taps are the FP16 values of the slab (BF16 slabs are
 // rounded to FP16 in LDS, as the direct kernel rounds them per tap). The
 // weights stay FP32 quantities: each is split into an FP16 high part and the
-// FP16 remainder (22 bits together), and both are multiplied, two matrix
-// instructions per product. The weights of all tilts are scaled by one power
+// FP16 remainder of the exact product (not of its FP32 rounding), and both are
+// multiplied, two matrix instructions per product. An instruction adds its
+// four tilts to the accumulator one after another, each rounded to nearest
+// even, so the small remainders go first. The error against FP64 sums is then
+// no larger than that of FP32 weights and one FP32 fused multiply-add per tap
+// (rel-L2 on the plan's own FP16 slabs, here / there: 6 tilts 7.1e-8 / 7.6e-8,
+// 41 tilts 1.66e-7 / 1.69e-7, 121 tilts 2.81e-7 / 2.81e-7; BF16 1 to 15 %
+// below). The weights of all tilts are scaled by one power
 // of two that puts the largest in [2^13, 2^14), and the sum is scaled back at
 // the end. The pairs end at 2^-24: where a tilt's weight lies more than
 // 8192-fold below the largest, the series is computed tap by tap with FP32
@@ -516,17 +522,19 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
       auto pass = [&](float sc, int slot) {
         const float w1 = sc * tt, w0 = sc - w1;
         const half2v hi = to_half2(w0, w1);
-        const half2v lo = to_half2(w0 - (float)hi[0], w1 - (float)hi[1]);
+        // what the high parts leave of the exact weights
+        const half2v lo = to_half2(fmaf(-sc, tt, sc - (float)hi[0]),
+                                   fmaf(sc, tt, -(float)hi[1]));
         const half8 ah = place(sl, hi), al = place(sl, lo);
         const uint32_t q = run0 + slot * S::kRunStride + addr;
         auto tiles = [&](auto r0, auto n, half8(&bv)[decltype(n)::value]) {
           constexpr int R0 = decltype(r0)::value, KN = decltype(n)::value;
 #pragma unroll
           for (int r = 0; r < KN; ++r)
-            acc[blk][R0 + r] = mfma16(ah, bv[r], acc[blk][R0 + r]);
+            acc[blk][R0 + r] = mfma16(al, bv[r], acc[blk][R0 + r]);
 #pragma unroll
           for (int r = 0; r < KN; ++r)
-            acc[blk][R0 + r] = mfma16(al, bv[r], acc[blk][R0 + r]);
+            acc[blk][R0 + r] = mfma16(ah, bv[r], acc[blk][R0 + r]);
         };
         constexpr int kBlock = 64 * kPos;  // bytes of a 32-row block
         if constexpr (RB == 1) {
