@@ -56,9 +56,9 @@
 // and one 1 KiB load covers whole 64-byte pieces of the slab.
 //
 // Exceptional values. A zero weight times a NaN or an infinity would reach
-// voxels that do not read it. A tile that ends with a value that is not
-// finite is therefore computed again tap by tap, so that such values reach
-// exactly the voxels that read them.
+// voxels that do not read it. The rows of a tile that end with a value that is
+// not finite are therefore computed again tap by tap, so that such values
+// reach exactly the voxels that read them; other rows keep their values.
 #include <type_traits>
 
 #include "gx_bp_geometry.hpp"
@@ -135,7 +135,7 @@ __device__ __forceinline__ int tile_of(unsigned lb, int nbx, int nbz, int &bx,
   return (int)grp;
 }
 
-// The same for two 32-row blocks.
+// read_tr8x2 for two 32-row blocks.
 template <int OFF, int STEP>
 __device__ __forceinline__ void read_tr8x4(uint32_t a, half8 &h0, half8 &h1,
                                            half8 &h2, half8 &h3) {
@@ -162,6 +162,31 @@ __device__ __forceinline__ void read_tr8x4(uint32_t a, half8 &h0, half8 &h1,
     *out[i] = __builtin_bit_cast(
         half8, __builtin_shufflevector(v[2 * i], v[2 * i + 1], 0, 1, 2, 3, 4,
                                        5, 6, 7));
+}
+
+// Eight rows of two positions, at LDS addresses a0 and a1, in each of N
+// 32-row blocks from OFF on, STEP bytes apart.
+template <int OFF, int STEP, int N>
+__device__ __forceinline__ void read_rows(uint32_t a0, uint32_t a1,
+                                          half8 (&v0)[N], half8 (&v1)[N]) {
+  if constexpr (N == 1)
+    asm volatile(
+        "ds_read_b128 %0, %2 offset:%4\n\t"
+        "ds_read_b128 %1, %3 offset:%4\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v0[0]), "=&v"(v1[0])
+        : "v"(a0), "v"(a1), "n"(OFF)
+        : "memory");
+  else
+    asm volatile(
+        "ds_read_b128 %0, %4 offset:%6\n\t"
+        "ds_read_b128 %1, %5 offset:%6\n\t"
+        "ds_read_b128 %2, %4 offset:%7\n\t"
+        "ds_read_b128 %3, %5 offset:%7\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v0[0]), "=&v"(v1[0]), "=&v"(v0[1]), "=&v"(v1[1])
+        : "v"(a0), "v"(a1), "n"(OFF), "n"(OFF + STEP)
+        : "memory");
 }
 
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
@@ -572,17 +597,60 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
     }
   };
 
+  // Each lane holds, per block and 16-row tile, 4 voxels in x (row m, z =
+  // g): 16 rows at a time pass through LDS and leave as 64-byte pieces.
+  auto store_all = [&]() {
+    const bool wide = W % 4 == 0 && (reinterpret_cast<uintptr_t>(vol) & 15) == 0;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int r = 0; r < kRT; ++r) {
+      float *out = reinterpret_cast<float *>(lds + (r & 1) * kBufWords);
 #pragma unroll
-    for (int r = 0; r < kRT; ++r) acc[i][r] = (float4v)(0.0f);
-  if (!taps) {
+      for (int i = 0; i < 2; ++i) {
+        float *q = out + m * S::kOutRow +
+                   (8 * (wave >> 2) + 4 * i + g) * kTile + 4 * (wave & 3);
+        float4v v = acc[i][r];
+        *reinterpret_cast<float4v *>(q) = v * down;
+      }
+      lds_barrier();
+      if (wide) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int row = 2 * wave + i;
+          const int y = byb * YB + 16 * r + row;
+          const int oz = bz * kTile + (lane >> 2);
+          const int ox = bx * kTile + 4 * (lane & 3);
+          if (y < Y && oz < Z && ox < W)
+            *reinterpret_cast<float4v *>(
+                vol + ((size_t)(y - y_base) * Z + oz) * W + ox) =
+                *reinterpret_cast<const float4v *>(out + row * S::kOutRow +
+                                                   4 * lane);
+        }
+      } else {
+        // lines of W values are not whole 16-byte words: a lane per voxel
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int row = 2 * wave + (i >> 2);
+          const int y = byb * YB + 16 * r + row;
+          const int oz = bz * kTile + 4 * (i & 3) + (lane >> 4);
+          const int ox = bx * kTile + (lane & 15);
+          if (y < Y && oz < Z && ox < W)
+            vol[((size_t)(y - y_base) * Z + oz) * W + ox] =
+                out[row * S::kOutRow + 64 * (i & 3) + lane];
+        }
+      }
+    }
+  };
+
+  // All batches through body(batch, its buffer): the next one's loads are
+  // issued first, into the other buffer. (One copy of the loop body: two, one
+  // for each buffer order, made the compiler keep the accumulators twice and
+  // spill.)
+  auto batches = [&](auto body) {
     Batch b = next_batch(0);
     stage(b, lds);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     convert(b, lds);
     lds_barrier();
-    // One batch: issue the next one's loads into `nxt`, multiply `cur`.
     auto step = [&](const uint4 *cur, uint4 *nxt) {
       const int t1 = b.t0 + b.nt;
       Batch nb{t1, 0, 0};
@@ -590,7 +658,7 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
         nb = next_batch(t1);
         stage(nb, nxt);
       }
-      multiply(b, cur);
+      body(b, cur);
       if (t1 < T) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         convert(nb, nxt);
@@ -598,127 +666,131 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
       lds_barrier();
       b = nb;
     };
-    // (one copy of the loop body: two, one for each buffer order, made the
-    // compiler keep the accumulators twice and spill)
     int odd = 0;
 #pragma unroll 1
     while (b.t0 < T) {
       step(lds + odd * kBufWords, lds + (1 - odd) * kBufWords);
       odd = 1 - odd;
     }
-  }
+  };
 
-  bool bad = taps;
-#pragma unroll
-  for (int r = 0; r < kRT; ++r) {
-    const bool row = byb * YB + 16 * r + m < Y;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        bad |= row && !(fabsf(acc[i][r][j]) < __builtin_inff());
-  }
-  if (__syncthreads_or(bad)) {
-    // Again, tap by tap on the vector units: lane (g, m) holds row m of
-    // voxels 4 g + i.
+  unsigned bad = 0;  // bit r: a value of row 16 r + m is not finite
+  bool redo = true;
+  if (!taps) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int r = 0; r < kRT; ++r) acc[i][r] = (float4v)(0.0f);
-#pragma unroll 1
-    for (int t0 = 0; t0 < T;) {
-      const Batch b = next_batch(t0);
-      stage(b, lds);
-      t0 += b.nt;
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      convert(b, lds);
-      lds_barrier();
-      float4 cf;
-      int2 w;
-      lane_tables(b, lds, cf, w);
-      const int exg = MULTI ? (b.ex >> (4 * g)) & 15 : 0;
+    batches(multiply);
 #pragma unroll
-      for (int blk = 0; blk < 2; ++blk) {
+    for (int r = 0; r < kRT; ++r) {
+      bool b = false;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          b |= !(fabsf(acc[i][r][j]) < __builtin_inff());
+      if (b && byb * YB + 16 * r + m < Y) bad |= 1u << r;
+    }
+    redo = __syncthreads_or((int)bad) != 0;
+    store_all();
+  }
+  if (!redo) return;
+
+  // The rows that are not finite, tap by tap on the vector units: FP32
+  // weights, the taps of exactly the voxels that read them, added in tilt
+  // order as k_bp_lds adds them. A thread takes two voxels (of z and z + 8)
+  // and 8 of every 32 rows; four neighbouring lanes share a voxel, so that 16
+  // lanes read four positions of all rows, 256 bytes in distinct banks.
+  // 61 corrected projections of 1024^2, a NaN in one (all rows, no matrix
+  // pass: k_bp_coefficients): 4.23 ms with a lane per row of its matrix tile
+  // and 2-byte LDS reads, 1.49 here, 1.27 with k_bp_lds. The results are stored
+  // over those of the matrix pass, once these have left.
+  __shared__ uint32_t rows_bad[RB];  // a bit per row
+  if (threadIdx.x < RB) rows_bad[threadIdx.x] = taps ? ~0u : 0u;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_barrier();
+#pragma unroll
+  for (int r = 0; r < kRT; ++r)
+    if ((bad >> r) & 1) atomicOr(&rows_bad[r >> 1], 1u << (16 * (r & 1) + m));
+  lds_barrier();
+  unsigned todo = 0;  // 32-row blocks with such rows
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+    if (rows_bad[i] != 0 && byb * YB + 32 * i < Y) todo |= 1u << i;
+  todo = (unsigned)__builtin_amdgcn_readfirstlane((int)todo);
+
+  const int part8 = (int)threadIdx.x & 3;  // rows 8 part8 .. of a block
+  const int vox = (int)threadIdx.x >> 2;
+  const int vx = bx * kTile + (vox & 15), vz = bz * kTile + (vox >> 4);
+  const float px = voxel_coord(min(vx, W - 1), W);
+  const float pz[2] = {voxel_coord(min(vz, Z - 1), Z),
+                       voxel_coord(min(vz + 8, Z - 1), Z)};
+  const int lane_off = (part8 >> 1) * 128 + (part8 & 1) * 16;
+  float sum[2][RB][8];
+#pragma unroll
+  for (int v = 0; v < 2; ++v)
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int r = 0; r < 8; ++r) sum[v][i][r] = 0.0f;
+  batches([&](const Batch &b, const uint4 *cur) {
+    const uint32_t run0 = lds_address(cur) + lane_off;
+#pragma unroll 1
+    for (int j = 0; j < b.nt; ++j) {
+      const float4 cf = kload(coef, b.t0 + j);
+      const int2 w = kload(tw, b.t0 + j);
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
         float tt;
-        const int i0 = tap_index<false>(x, zb[blk], cf, tt);
-        const int ok = (unsigned)i0 < (unsigned)(N - 1);
-        const int rel = min(max(i0 - w.x, 0), kPos - 2);
-        int slot = g;
-        if constexpr (MULTI) {
-          const int kr = min(max(slab_of(x, zb[blk], cf, dscale, doffset,
-                                         ndf) - (w.y & kSlabMask), 0),
-                             w.y >> kSpanShift);
-          slot = kr == 0 ? g : 3 + exg + kr;
-        }
-#pragma unroll 1
-        for (int tg = 0; tg < b.nt; ++tg) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int from = 16 * tg + 4 * g + i;
-            const float ft = __shfl(tt, from), fw = __shfl(cf.w, from);
-            const int p0 = __shfl(rel, from), p1 = p0 + 1;
-            const int fs = __shfl(slot, from);
-            const bool fok = __shfl(ok, from) != 0;
-            const float w1 = fw * ft, w0 = fw - w1;
-            const char *q = reinterpret_cast<const char *>(lds) +
-                            fs * S::kRunStride + m * 2;
-            const int o0 = (p0 >> 2) * 256 + (p0 & 3) * 32;
-            const int o1 = (p1 >> 2) * 256 + (p1 & 3) * 32;
-#pragma unroll
-            for (int r = 0; r < kRT; ++r) {
-              const char *qr = q + (r >> 1) * (64 * kPos) + (r & 1) * 128;
-              const float v0 = *reinterpret_cast<const _Float16 *>(qr + o0);
-              const float v1 = *reinterpret_cast<const _Float16 *>(qr + o1);
-              const float s = fmaf(w1, v1, fmaf(w0, v0, acc[blk][r][i]));
-              acc[blk][r][i] = fok ? s : acc[blk][r][i];
+        const int i0 = tap_index<false>(px, pz[v], cf, tt);
+        if ((unsigned)i0 < (unsigned)(N - 1)) {
+          int slot = j;
+          if constexpr (MULTI) {
+            // (a tile within one slab at a tilt has its own run alone)
+            if (w.y >> kSpanShift) {
+              const int kr =
+                  min(max(slab_of(px, pz[v], cf, dscale, doffset, ndf) -
+                              (w.y & kSlabMask), 0), w.y >> kSpanShift);
+              if (kr > 0) slot = 3 + ((b.ex >> (4 * j)) & 15) + kr;
             }
           }
+          const int p0 = min(max(i0 - w.x, 0), kPos - 2), p1 = p0 + 1;
+          const uint32_t q = run0 + slot * S::kRunStride;
+          const uint32_t a0 = q + (p0 >> 2) * 256 + (p0 & 3) * 32;
+          const uint32_t a1 = q + (p1 >> 2) * 256 + (p1 & 3) * 32;
+          const float w1 = cf.w * tt, w0 = cf.w - w1;
+          auto blocks = [&](auto i, auto n) {
+            constexpr int I = decltype(i)::value, KN = decltype(n)::value;
+            constexpr int kBlock = 64 * kPos;
+            if (((todo >> I) & ((1u << KN) - 1)) == 0) return;
+            half8 v0[KN], v1[KN];
+            read_rows<I * kBlock, kBlock>(a0, a1, v0, v1);
+#pragma unroll
+            for (int k = 0; k < KN; ++k)
+#pragma unroll
+              for (int r = 0; r < 8; ++r)
+                sum[v][I + k][r] =
+                    fmaf(w1, (float)v1[k][r],
+                         fmaf(w0, (float)v0[k][r], sum[v][I + k][r]));
+          };
+          blocks(Int<0>(), Int<(RB > 1 ? 2 : 1)>());
+          if constexpr (RB > 2) blocks(Int<2>(), Int<2>());
         }
       }
-      lds_barrier();
     }
-  }
-
-  // Each lane holds, per block and 16-row tile, 4 voxels in x (row m, z =
-  // g): 16 rows at a time pass through LDS and leave as 64-byte pieces.
-  const bool wide = W % 4 == 0 && (reinterpret_cast<uintptr_t>(vol) & 15) == 0;
+  });
 #pragma unroll
-  for (int r = 0; r < kRT; ++r) {
-    float *out = reinterpret_cast<float *>(lds + (r & 1) * kBufWords);
+  for (int i = 0; i < RB; ++i) {
+    const uint32_t rows8 = rows_bad[i] >> (8 * part8);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float *q = out + m * S::kOutRow +
-                 (8 * (wave >> 2) + 4 * i + g) * kTile + 4 * (wave & 3);
-      float4v v = acc[i][r];
-      *reinterpret_cast<float4v *>(q) = v * down;
-    }
-    lds_barrier();
-    if (wide) {
+    for (int v = 0; v < 2; ++v)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int row = 2 * wave + i;
-        const int y = byb * YB + 16 * r + row;
-        const int oz = bz * kTile + (lane >> 2);
-        const int ox = bx * kTile + 4 * (lane & 3);
-        if (y < Y && oz < Z && ox < W)
-          *reinterpret_cast<float4v *>(
-              vol + ((size_t)(y - y_base) * Z + oz) * W + ox) =
-              *reinterpret_cast<const float4v *>(out + row * S::kOutRow +
-                                                 4 * lane);
+      for (int r = 0; r < 8; ++r) {
+        const int y = byb * YB + 32 * i + 8 * part8 + r, oz = vz + 8 * v;
+        if (((rows8 >> r) & 1) && y < Y && oz < Z && vx < W)
+          vol[((size_t)(y - y_base) * Z + oz) * W + vx] = sum[v][i][r];
       }
-    } else {
-      // lines of W values are not whole 16-byte words: a lane per voxel
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int row = 2 * wave + (i >> 2);
-        const int y = byb * YB + 16 * r + row;
-        const int oz = bz * kTile + 4 * (i & 3) + (lane >> 4);
-        const int ox = bx * kTile + (lane & 15);
-        if (y < Y && oz < Z && ox < W)
-          vol[((size_t)(y - y_base) * Z + oz) * W + ox] =
-              out[row * S::kOutRow + 64 * (i & 3) + lane];
-      }
-    }
   }
 }
 

@@ -308,6 +308,10 @@ __global__ __launch_bounds__(RP * (X / default_e(X))) void k_rows_r2c(
   // a pair of rows is one wave (or part of one) up to 1024 points: its
   // transform synchronises only that wave
   Fft<X, E, -1, 1, (NT <= 64)>::run(v, s[p], tid, tw);
+  // A NaN of these rows is in every output now, and the correction takes it
+  // to the whole projection, whatever its scale: infinity as the largest
+  // value tells the backprojection.
+  if (__builtin_isunordered(v[0].x, v[0].y)) amax = __builtin_inff();
 #pragma unroll
   for (int m = 0; m < E; ++m) s[p][tid + m * NT] = v[m];
   lds_barrier();
@@ -1282,6 +1286,8 @@ __global__ __launch_bounds__(P * (M / default_e(M))) void k_rows_r2c_bs(
     amax = fmaxf(amax, fmaxf(fabsf(a), fabsf(b)));
   }
   bluestein<M, E, -1, 1>(v, s[p], tid, twm, bx);
+  // (a NaN, as in k_rows_r2c)
+  if (__builtin_isunordered(v[0].x, v[0].y)) amax = __builtin_inff();
 #pragma unroll
   for (int m = 0; m < E; ++m) {
     const int n = tid + m * NT;
