@@ -809,7 +809,11 @@ static hipError_t launch_bp_lds_k(const BpArgs &a, hipStream_t s) {
 
 template <int YB, int STORE>
 static hipError_t launch_bp_lds_t(const BpArgs &a, hipStream_t s) {
-  if (a.ndf == 1) return launch_bp_lds_k<YB, STORE, false, 1>(a, s);
+  if (a.ndf == 1) {
+    if constexpr (STORE == kF32)
+      return launch_bp_lds_k<YB, STORE, false, 1>(a, s);
+    return hipErrorInvalidValue;  // 16 bits, one slab: launch_bp_mm
+  }
   switch (a.staged) {
     case 2: return launch_bp_lds_k<YB, STORE, true, 2>(a, s);
     case 4: return launch_bp_lds_k<YB, STORE, true, 4>(a, s);
@@ -830,11 +834,13 @@ static hipError_t launch_bp_t(const BpArgs &a, hipStream_t s) {
                        s, (const ST *)a.slab, a.coef, a.dscale, a.doffset,
                        a.ndf, a.N, a.T, a.NYB, a.W, a.Z, a.Y, a.yb0, a.y_base, a.slab_yb0,
                        a.vol, nbx, nbz, nb);
-  } else {
+  } else if constexpr (STORE == kF32) {
     hipLaunchKernelGGL((k_bp<YB, STORE, false>), dim3(nb), dim3(kTX * kTZ), 0,
                        s, (const ST *)a.slab, a.coef, a.dscale, a.doffset,
                        a.ndf, a.N, a.T, a.NYB, a.W, a.Z, a.Y, a.yb0, a.y_base, a.slab_yb0,
                        a.vol, nbx, nbz, nb);
+  } else {
+    return hipErrorInvalidValue;  // 16 bits, one slab: launch_bp_mm
   }
   return hipGetLastError();
 }

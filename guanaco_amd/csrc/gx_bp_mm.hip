@@ -46,14 +46,15 @@
 // LDS. Per (tilt, slab) a run of kPos = 24 positions of the tile's rows is
 // loaded straight into LDS (the tile's taps span 15 |c| + 15 |s| <= 21.22
 // positions), four tilts to a batch, two buffers: the loads of a batch are
-// issued before the one before it is multiplied. A tile that spans more
-// slabs at a tilt takes extra runs (two per batch; a batch closes early when
-// they do not suffice). The matrix operand needs 8 positions of one row in
-// each lane, while a slab holds the rows of a position contiguously: the
-// transposing LDS read (ds_read_b64_tr_b16) does that. Runs are laid out
-// [32-row block][4 positions][16-row half][position][16 rows], so that one
-// read of 16 lanes is 4 consecutive positions x 32 bytes in distinct banks
-// and one 1 KiB load covers whole 64-byte pieces of the slab.
+// issued before the one before it is multiplied. A tile that spans two slabs
+// at a tilt (two at most: they are 64 pixels or wider) takes a second run; a
+// batch holds two of these and closes early for a third. The matrix operand
+// needs 8 positions of one row in each lane, while a slab holds the rows of a
+// position contiguously: the transposing LDS read (ds_read_b64_tr_b16) does
+// that. Runs are laid out [32-row block][4 positions][16-row half][position]
+// [16 rows], so that one read of 16 lanes is 4 consecutive positions x 32
+// bytes in distinct banks and one 1 KiB load covers whole 64-byte pieces of
+// the slab.
 //
 // Exceptional values. A zero weight times a NaN or an infinity would reach
 // voxels that do not read it. The rows of a tile that end with a value that is
@@ -72,13 +73,13 @@ namespace {
 constexpr int kTile = 16;    // voxels of a tile in x and in z
 constexpr int kPos = 24;     // staged positions
 constexpr int kMaxBase = kPos - 8;
-constexpr int kExtra = 2;    // runs of second and third slabs per batch
+constexpr int kExtra = 2;    // runs of second slabs per batch
 constexpr int kWaves = 8;
 // order of the tiles (tile_of)
 constexpr unsigned kStrip = 8;
 constexpr unsigned kWhole = 16;
 constexpr size_t kFill = 256;
-// window table: .y = first slab | (slabs - 1) << kSpanShift
+// window table: .y = first slab | (1 where there are two) << kSpanShift
 constexpr int kSpanShift = 28;
 constexpr int kSlabMask = (1 << kSpanShift) - 1;
 
@@ -289,7 +290,7 @@ __global__ void k_bp_mm_windows(const float4 *__restrict__ coef, int T,
         k1 = max(k1, k);
       }
     }
-    r = make_int2(w, MULTI ? k0 | (min(k1 - k0, kExtra) << kSpanShift) : 0);
+    r = make_int2(w, MULTI ? k0 | (min(k1 - k0, 1) << kSpanShift) : 0);
   }
   win[i] = r;
 }
@@ -580,19 +581,22 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
       if constexpr (!MULTI) {
         pass(s, g);
       } else {
-        // One pass per slab that some voxel of the block's tilt reads: each
-        // group of 16 lanes (one tilt) takes its smallest slab left.
-        bool left = true;
-        do {
-          int ks = 0;
-          bool take = left;
-          if (b.ex >> 16) {
-            ks = min16(left ? kr : kExtra + 1);
-            take = left && kr == ks;
-          }
-          pass(take ? s : 0.0f, ks == 0 || ks > kExtra ? g : 3 + exg + ks);
-          left = left && !take;
-        } while (__ballot(left) != 0);
+        // One pass, or two: each group of 16 lanes (one tilt) takes the
+        // first slab that a voxel of the block reads, then the second one.
+        int ks = 0;
+        if (b.ex >> 16) ks = min16(kr);
+        float sc = kr == ks ? s : 0.0f;
+        int slot = ks != 0 ? 4 + exg : g;
+        bool left = kr != ks;
+#pragma unroll 1
+        for (;;) {
+          pass(sc, slot);
+          if (__ballot(left) == 0) break;
+          // (a tile within one slab at a tilt has no second run)
+          sc = left ? s : 0.0f;
+          slot = w.y >> kSpanShift ? 4 + exg : g;
+          left = false;
+        }
       }
     }
   };
@@ -748,12 +752,10 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void k_bp_mm(
           int slot = j;
           if constexpr (MULTI) {
             // (a tile within one slab at a tilt has its own run alone)
-            if (w.y >> kSpanShift) {
-              const int kr =
-                  min(max(slab_of(px, pz[v], cf, dscale, doffset, ndf) -
-                              (w.y & kSlabMask), 0), w.y >> kSpanShift);
-              if (kr > 0) slot = 3 + ((b.ex >> (4 * j)) & 15) + kr;
-            }
+            if (w.y >> kSpanShift &&
+                slab_of(px, pz[v], cf, dscale, doffset, ndf) >
+                    (w.y & kSlabMask))
+              slot = 4 + ((b.ex >> (4 * j)) & 15);
           }
           const int p0 = min(max(i0 - w.x, 0), kPos - 2), p1 = p0 + 1;
           const uint32_t q = run0 + slot * S::kRunStride;

@@ -156,7 +156,7 @@ hipError_t launch_bp_windows(const float4 *coef, int exact, int T, int W,
                              int2 *win, hipStream_t s);
 
 // The matrix-core kernel of 16-bit slabs (one centre, a 16 x 16 tile spans at
-// most three slabs; a.win from launch_bp_mm_windows): any rows per block YB
+// most two slabs; a.win from launch_bp_mm_windows): any rows per block YB
 // that the storage has. bp_mm_suits: the plans it is the faster kernel for.
 bool bp_mm_suits(int ndf, float dscale, int W, int Z, int Y);
 hipError_t launch_bp_mm(const BpArgs &a, int YB, int store, hipStream_t s);
