@@ -139,9 +139,9 @@ def correct_projections(projections, centre=None, pixel_size=1, energy=None,
                   Pa=astigmatism_angle * pi / 180, phi=phase_shift * pi / 180)
     defoci = [float(mn + d * step) for d in range(ndf)]
     # blocks of tilts of about 256 MiB of results, written in place where the
-    # output is plain float32 memory
-    n = max(1, (256 << 20) // (4 * ndf * Y * X))
-    direct = (isinstance(corrected, numpy.ndarray)
+    # output is plain float32 memory (a subclass may keep more than its values)
+    n = max(1, (256 << 20) // max(1, 4 * ndf * Y * X))
+    direct = (type(corrected) in (numpy.ndarray, numpy.memmap)
               and corrected.dtype == numpy.float32
               and corrected.flags.c_contiguous and corrected.flags.writeable)
     for z in range(0, T, n):
