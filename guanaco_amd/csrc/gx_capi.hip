@@ -903,11 +903,15 @@ std::string device_model() {
   return names[dev];
 }
 
+// (the last field tells plans of one shape by what their backprojector holds
+// per tilt: the staged kernel's slabs, 10 more on the matrix cores, which
+// depends on the width of the slabs)
 std::string tune_key(const gx_volume_plan *p) {
   char b[256];
   std::snprintf(b, sizeof b, "%s %d %d %d %d %d %d %d %d %d %d",
                 device_model().c_str(), p->X, p->Y, p->T, p->ndf, p->Z, p->W,
-                p->storage, p->layout, p->ctf ? 1 : 0, p->bp_staged);
+                p->storage, p->layout, p->ctf ? 1 : 0,
+                p->bp_staged + (p->bp_mm ? 10 : 0));
   return b;
 }
 
