@@ -278,7 +278,8 @@ def measure_path(C, w, angles, d_in, d_vol, stream, storage, graph, steps,
                  value=updates / (ms * 1e-3), p50_ms=percentile(lat, 50),
                  p99_ms=percentile(lat, 99), wall_s=wall, filter_ms=filt_ms,
                  bp_ms=bp_ms, bp_updates_per_s=updates / (bp_ms * 1e-3),
-                 backprojector=("staged, %d slab(s) per tilt" % slots
+                 backprojector=("matrix cores" if plan.matrix_cores() else
+                                "staged, %d slab(s) per tilt" % slots
                                 if kind == C.BP_STAGED else "direct"),
                  tile_rows=plan.tile()[0], launch="graph" if graph
                  else "eager", band_rows=band if band < Y else None,
@@ -641,10 +642,10 @@ def load_counters(name):
     return out
 
 
-def bp_kernel(storage):
-    """The backprojection kernel of a workload's plans: the matrix-core
-    kernel for 16-bit slabs (every workload here is in its range)."""
-    return "k_bp_mm" if storage in ("f16", "bf16") else "k_bp_lds"
+def bp_kernel(entry):
+    """The backprojection kernel of a measured path."""
+    return ("k_bp_mm" if entry["backprojector"] == "matrix cores"
+            else "k_bp_lds")
 
 
 def bp_roofline(w, entry, counters):
@@ -670,7 +671,7 @@ def bp_roofline(w, entry, counters):
     roof = {
         "bound": "hbm",
         "kernel": "%s (backprojection, %s slabs)" % (
-            bp_kernel(entry["storage"]), entry["storage"]),
+            bp_kernel(entry), entry["storage"]),
         "achieved": achieved,
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
@@ -867,7 +868,7 @@ def main():
                                        True)
     head = entry["paths"]["batched"]
     counters = load_counters("counters_%s_bp.txt" % args.config).get(
-        "%s %s" % (bp_kernel(head["storage"]), head["storage"]), {})
+        "%s %s" % (bp_kernel(head), head["storage"]), {})
     if counters:
         counters["_file"] = "counters_%s_bp.txt" % args.config
     line = {

@@ -196,6 +196,7 @@ SIGNATURES = {
     "gx_volume_plan_set_backprojector": [_vp, _int],
     "gx_volume_plan_get_backprojector": [_vp, ctypes.POINTER(_int),
                                          ctypes.POINTER(_int)],
+    "gx_volume_plan_matrix_cores": [_vp, ctypes.POINTER(_int)],
     "gx_volume_plan_slab_range": [_vp, ctypes.POINTER(_int),
                                   ctypes.POINTER(_int)],
     "gx_volume_slabs": [_vp, ctypes.POINTER(_vp), ctypes.POINTER(_sz),
@@ -507,6 +508,13 @@ class VolumePlan:
         call("gx_volume_plan_get_backprojector", self.handle, ctypes.byref(k),
              ctypes.byref(n))
         return k.value, n.value
+
+    def matrix_cores(self):
+        """Whether the backprojection runs on the matrix cores (whatever
+        backprojector() says: both kinds then stand for that kernel)."""
+        yes = _int()
+        call("gx_volume_plan_matrix_cores", self.handle, ctypes.byref(yes))
+        return bool(yes.value)
 
     def tile(self):
         """(rows per backprojection tile, backprojector kind)."""

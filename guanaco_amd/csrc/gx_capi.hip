@@ -1487,6 +1487,12 @@ extern "C" int gx_volume_plan_get_backprojector(gx_volume_plan *p, int *kind,
   return GX_OK;
 }
 
+extern "C" int gx_volume_plan_matrix_cores(gx_volume_plan *p, int *yes) {
+  GX_CHECK(p != nullptr && yes != nullptr);
+  *yes = p->bp_mm ? 1 : 0;
+  return GX_OK;
+}
+
 extern "C" int gx_volume_rows_per_block(gx_volume_plan *p, size_t *rows) {
   GX_CHECK(p != nullptr && rows != nullptr);
   *rows = (size_t)p->YB;

@@ -280,6 +280,8 @@ int gx_volume_rows_per_block(gx_volume_plan *plan, size_t *rows);
 int gx_volume_plan_set_backprojector(gx_volume_plan *plan, int kind);
 int gx_volume_plan_get_backprojector(gx_volume_plan *plan, int *kind,
                                      int *slabs_per_tilt);
+/* Whether the plan's backprojection runs on the matrix cores. */
+int gx_volume_plan_matrix_cores(gx_volume_plan *plan, int *yes);
 /* The plan's filtered slabs: [k][t][y/YB][x][y%YB], element size by storage.
  * Plans with several defocus slabs compute, at each tilt t, only the slabs
  * [first[t], last[t]] that some voxel of the volume reads (no reference

@@ -30,6 +30,7 @@ def run_plan(shape, storage, rows, sino, weights=None):
                         centre=X / 2.0 - 0.3, min_defocus=mn, max_defocus=mx,
                         weights=weights, storage=storage,
                         input_layout=C.INPUT_SINOGRAMS)
+    assert plan.matrix_cores()
     plan.set_tile(rows, "staged")
     d_in = C.DeviceArray.from_host(sino)
     d_vol = C.DeviceArray((Y, Z, W))

@@ -62,6 +62,7 @@ def test_no_further_off_than_fp32(capi, case, storage):
     plan = C.VolumePlan(X, Y, angles, Z, width=W, num_defocus=ndf,
                         centre=X / 2.0 - 0.3, min_defocus=mn, max_defocus=mx,
                         storage=storage, input_layout=C.INPUT_SINOGRAMS)
+    assert plan.matrix_cores()
     d_in = C.DeviceArray.from_host(sino)
     d_vol = C.DeviceArray((Y, Z, W))
     plan.run(d_in, d_vol)

@@ -56,6 +56,7 @@ def test_weak_tilts_keep_their_precision(capi, shape, kind, storage):
     plan = C.VolumePlan(X, Y, angles, Z, width=W, num_defocus=ndf,
                         centre=X / 2.0 - 0.3, min_defocus=mn, max_defocus=mx,
                         storage=storage, input_layout=C.INPUT_SINOGRAMS)
+    assert plan.matrix_cores()
     d_in = C.DeviceArray.from_host(sino)
     d_vol = C.DeviceArray((Y, Z, W))
     plan.run(d_in, d_vol)
