@@ -77,7 +77,7 @@ constexpr int kExtra = 2;    // runs of second slabs per batch
 constexpr int kWaves = 8;
 // order of the tiles (tile_of)
 constexpr unsigned kStrip = 8;
-constexpr unsigned kWhole = 16;
+constexpr unsigned kDeep = 32, kWide = 96;
 constexpr size_t kFill = 256;
 // window table: .y = first slab | (1 where there are two) << kSpanShift
 constexpr int kSpanShift = 28;
@@ -115,17 +115,22 @@ __device__ __forceinline__ void read_tr8x2(uint32_t a, half8 &h0, half8 &h1) {
 }
 
 // Tile of block lb, and its row group (returned). The 64 tiles an XCD runs at
-// a time share its L2: in a deep volume they are 8 x 8 (strips of 8 tiles in
-// z, along x), whose taps of a tilt span 128 (|c| + |s|) positions at most, not
-// one column of tiles through the depth, 16 |c| + Z |s|. 121 tilts, 4096 x
-// 1024 x 4096 voxels, 32 slabs: 205 -> 140 GB fetched; 61 tilts, 2048 x 512 x
-// 2048, 16 slabs: whole step 18.2 -> 17.6 ms. Up to kWhole tiles of depth
-// (256 voxels) the columns are short enough, and walking x once beats reading
-// the slabs again for a second strip: 41 tilts, 1024 x 256 x 512, 4 slabs,
-// BF16: 715 us in columns, 740 in strips; one slab: no difference.
+// a time share its L2: in a deep, wide volume they are 8 x 8 (strips of 8
+// tiles in z, along x), whose taps of a tilt span 128 (|c| + |s|) positions at
+// most, not one column of tiles through the depth, 16 |c| + Z |s|: 121 tilts,
+// 4096 x 1024 x 4096 voxels, 32 slabs, 205 -> 140 GB fetched. Elsewhere a
+// column's slab rows stay in the caches anyway, and walking x once beats
+// reading them again for every strip. The time of strips over that of
+// columns, 61 tilts: 512 wide 0.96 to 1.02 (192 to 512 deep); 1024 wide, one
+// slab, 1.04 to 1.14 (272 to 1024 deep), 16 slabs 1.04 (272) to 0.97 (512);
+// 1536 wide, 4 slabs, 1.05 (272), 0.99 (512), 0.96 (1536); 2048 wide 1.02 to
+// 1.11 (272), 0.97 to 0.99 (512), 0.93 to 1.03 (1536 and 2048); 3072 wide
+// 1.06 to 1.14 (272), 0.91 to 0.98 (2048 and 3072).
 __device__ __forceinline__ int tile_of(unsigned lb, int nbx, int nbz, int &bx,
                                        int &bz) {
-  const unsigned nz = (unsigned)nbz, strip = nz > kWhole ? kStrip : nz;
+  const unsigned nz = (unsigned)nbz;
+  const unsigned strip =
+      nz >= kDeep && (unsigned)nbx >= kWide ? kStrip : nz;
   const unsigned nt = (unsigned)nbx * nz;
   const unsigned grp = lb / nt, r = lb - grp * nt;
   const unsigned s = r / (strip * (unsigned)nbx);

@@ -59,11 +59,22 @@ def test_row_groups(capi, shape, storage, rows):
     vol, taps = run_plan(shape, storage, rows, sino)
     nrm = numpy.abs(sino).max(axis=(0, 1, 3))
     slabs = taps * nrm[None, :, None, None]
-    for y in sorted({0, Y // 2, Y // 32 * 32 - 1, Y - 1}):
+    for y in sorted({0, Y // 2, max(Y // 32 * 32, 1) - 1, Y - 1}):
         expect = backproject(slabs[:, :, y], Z, W, ANGLES, X / 2.0 - 0.3, mn,
                              mx)
         err = numpy.linalg.norm(vol[y] - expect)
         assert err <= 1e-5 * numpy.linalg.norm(expect), (y, err)
+
+
+# depths and widths about the limits of the tile order (32 tiles deep and 96
+# wide): columns, strips of 8 tiles, a last strip of 1 and of 6, two row groups
+@pytest.mark.parametrize("shape", [
+    (60, 2, 1, 496, 1540, (0.0, 0.0)), (60, 2, 1, 513, 1520, (0.0, 0.0)),
+    (60, 2, 1, 512, 1521, (0.0, 0.0)), (60, 2, 1, 521, 1540, (0.0, 0.0)),
+    (60, 129, 1, 600, 1540, (0.0, 0.0)), (700, 2, 3, 513, 1536, (-300., 300.)),
+])
+def test_tile_orders(capi, shape):
+    test_row_groups(capi, shape, "f16", 32)
 
 
 @pytest.mark.parametrize("storage,rows", [("f16", 16), ("bf16", 32)])
