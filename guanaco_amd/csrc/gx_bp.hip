@@ -490,10 +490,12 @@ __device__ __forceinline__ typename StoreT<STORE>::T buffer_tap(
 // little read the same or the next position, so a load of a wave touches a
 // handful of cache lines. (With a lane per voxel, as in k_bp, each load
 // touched one line per lane and the address unit bound the kernel: 61 tilts,
-// 512 x 128 x 512 voxels, FP32: 4.94 ms; here 0.78.) A thread keeps 4 (x) by YB / 4 (z)
-// voxels; a workgroup is the same 32 x 8 voxels by YB rows. What binds it now
-// is vector issue, 17 instructions for an update: position, floor and
-// fraction, address, range and the reference's five roundings, none of which
+// 512 x 128 x 512 voxels, FP32: 4.94 ms; here 1.66e6 cycles, 0.69 ms at 2.4
+// GHz.) A thread keeps 4 (x) by YB / 4 (z) voxels; a workgroup is the same
+// 32 x 8 voxels by YB rows. The address and data units are busy 0.95 of that
+// time, 6 cycles for each of the two loads of a wave's updates, and the vector
+// units issue 15.7 instructions for an update: position, floor and fraction,
+// address, range and the reference's five roundings, none of which
 // rows share. A tile within one slab at a tilt (win) takes one buffer for
 // all its voxels; elsewhere each voxel chooses its slab.
 template <int YB, int STORE, bool MULTI>
