@@ -32,6 +32,7 @@
 namespace gx {
 
 constexpr int kTX = 32, kTZ = 8;
+constexpr size_t kRowTiles = 2048;  // (launch_bp_rows_t)
 
 template <int YB, int STORE>
 struct Taps;
@@ -491,14 +492,14 @@ __device__ __forceinline__ typename StoreT<STORE>::T buffer_tap(
 // handful of cache lines. (With a lane per voxel, as in k_bp, each load
 // touched one line per lane and the address unit bound the kernel: 61 tilts,
 // 512 x 128 x 512 voxels, FP32: 4.94 ms; here 1.66e6 cycles, 0.69 ms at 2.4
-// GHz.) A thread keeps 4 (x) by YB / 4 (z) voxels; a workgroup is the same
-// 32 x 8 voxels by YB rows. The address and data units are busy 0.95 of that
+// GHz.) A thread keeps 4 (x) by VZ (z) voxels; a workgroup is the same 32 x 8
+// voxels by YB rows (VZ = YB / 4) or a part of them. The address and data units are busy 0.95 of that
 // time, 6 cycles for each of the two loads of a wave's updates, and the vector
 // units issue 15.7 instructions for an update: position, floor and fraction,
 // address, range and the reference's five roundings, none of which
 // rows share. A tile within one slab at a tilt (win) takes one buffer for
 // all its voxels; elsewhere each voxel chooses its slab.
-template <int YB, int STORE, bool MULTI>
+template <int YB, int STORE, bool MULTI, int VZ>
 __global__ __launch_bounds__(kTX *kTZ) void k_bp_rows(
     const typename StoreT<STORE>::T *__restrict__ slab,
     const float4 *__restrict__ coef, const int2 *__restrict__ win,
@@ -508,14 +509,19 @@ __global__ __launch_bounds__(kTX *kTZ) void k_bp_rows(
     unsigned nblocks) {
   constexpr bool kExact = STORE == kF32;
   using ST = StoreT<STORE>;
-  constexpr int VX = 4, VZ = YB / 4;  // voxels of a thread
+  constexpr int VX = 4;               // (x) by VZ (z) voxels of a thread
   constexpr int GX = kTX / VX;        // thread groups of a tile in x
-  const unsigned lb = xcd_remap(blockIdx.x, nblocks);
+  constexpr int DZ = 32 * VZ / YB;    // z of a workgroup: kTZ, or a part
+  static_assert(kTZ % DZ == 0, "workgroups split a tile");
+  constexpr unsigned kParts = kTZ / DZ;
+  const unsigned lp = xcd_remap(blockIdx.x, nblocks);
+  const unsigned lb = lp / kParts, part = lp % kParts;
   const int bz = (int)(lb % (unsigned)nbz);
   const int bx = (int)((lb / (unsigned)nbz) % (unsigned)nbx);
   const int byb = yb0 + (int)(lb / ((unsigned)nbz * (unsigned)nbx));
   const int r = (int)threadIdx.x % YB, q = (int)threadIdx.x / YB;
-  const int ix = bx * kTX + (q % GX) * VX, iz = bz * kTZ + (q / GX) * VZ;
+  const int ix = bx * kTX + (q % GX) * VX;
+  const int iz = bz * kTZ + (int)part * DZ + (q / GX) * VZ;
   const int y = byb * YB + r;
   float x[VX], z[VZ];
 #pragma unroll
@@ -847,28 +853,45 @@ static hipError_t launch_bp_t(const BpArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <int YB, int STORE, bool MULTI, int VZ>
+static hipError_t launch_bp_rows_v(const BpArgs &a, size_t tiles,
+                                   hipStream_t s) {
+  using ST = typename StoreT<STORE>::T;
+  const size_t nb = tiles * (YB / 4 / VZ);
+  if (nb > 0xffffffffu) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_bp_rows<YB, STORE, MULTI, VZ>), dim3((unsigned)nb),
+                     dim3(kTX * kTZ), 0, s, (const ST *)a.slab, a.coef, a.win,
+                     a.row_off, a.Y_tab, a.dscale, a.doffset, a.ndf, a.N, a.T,
+                     a.NYB, a.W, a.Z, a.Y, a.yb0, a.y_base, a.slab_yb0, a.vol,
+                     (a.W + kTX - 1) / kTX, (a.Z + kTZ - 1) / kTZ,
+                     (unsigned)nb);
+  return hipGetLastError();
+}
+
+// A thread takes 4 x YB / 4 voxels, or 4 x 1, of which a tile needs YB / 4
+// workgroups: in a small volume few waves run, one after another of a thread's
+// loads is waited for, and a partial row block leaves lanes idle. 41 tilts,
+// backprojection alone, 4 x 1 over 4 x YB / 4 (and over a lane per voxel
+// column): up to 16 tiles times row blocks 0.09 to 0.40 (0.13 to 0.65; without
+// it 16-bit slabs took up to 5 times as long), 512 of them 0.33 to 1.04, 2048
+// 0.96 to 1.03 (0.14 to 0.71), from 4096 on 1.00 to 1.19. With several 16-bit
+// slabs at every size: 0.39 to 0.82 where neighbouring rows' centres lie
+// close, 0.96 to 1.01 where they do not.
 template <int YB, int STORE>
 static hipError_t launch_bp_rows_t(const BpArgs &a, hipStream_t s) {
-  using ST = typename StoreT<STORE>::T;
-  const int nbx = (a.W + kTX - 1) / kTX;
-  const int nbz = (a.Z + kTZ - 1) / kTZ;
   if (a.yb1 <= a.yb0) return hipSuccess;
-  const unsigned nb =
-      (unsigned)nbx * (unsigned)nbz * (unsigned)(a.yb1 - a.yb0);
+  const size_t tiles = (size_t)((a.W + kTX - 1) / kTX) *
+                       ((a.Z + kTZ - 1) / kTZ) * (a.yb1 - a.yb0);
   if (a.ndf > 1) {
-    hipLaunchKernelGGL((k_bp_rows<YB, STORE, true>), dim3(nb),
-                       dim3(kTX * kTZ), 0, s, (const ST *)a.slab, a.coef,
-                       a.win, a.row_off, a.Y_tab, a.dscale, a.doffset, a.ndf, a.N,
-                       a.T, a.NYB, a.W, a.Z, a.Y, a.yb0, a.y_base, a.slab_yb0, a.vol,
-                       nbx, nbz, nb);
-  } else {
-    hipLaunchKernelGGL((k_bp_rows<YB, STORE, false>), dim3(nb),
-                       dim3(kTX * kTZ), 0, s, (const ST *)a.slab, a.coef,
-                       a.win, a.row_off, a.Y_tab, a.dscale, a.doffset, a.ndf, a.N,
-                       a.T, a.NYB, a.W, a.Z, a.Y, a.yb0, a.y_base, a.slab_yb0, a.vol,
-                       nbx, nbz, nb);
+    if constexpr (STORE == kF32) {
+      if (tiles > kRowTiles)
+        return launch_bp_rows_v<YB, STORE, true, YB / 4>(a, tiles, s);
+    }
+    return launch_bp_rows_v<YB, STORE, true, 1>(a, tiles, s);
   }
-  return hipGetLastError();
+  if (tiles > kRowTiles)
+    return launch_bp_rows_v<YB, STORE, false, YB / 4>(a, tiles, s);
+  return launch_bp_rows_v<YB, STORE, false, 1>(a, tiles, s);
 }
 
 hipError_t launch_bp(const BpArgs &a, int YB, int store, hipStream_t s) {
