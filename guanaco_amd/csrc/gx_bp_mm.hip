@@ -835,21 +835,33 @@ static hipError_t launch_mm_rows(const BpArgs &a, hipStream_t s) {
   return launch_mm<YB, STORE, MULTI, 1>(a, s);
 }
 
-// With one slab always. With several, a workgroup's batches wait for window
-// entries and extra runs in turn, which takes other workgroups to hide and
-// wide slabs to be rare: two workgroups per CU (512) and slabs of at least 64
-// pixels. Measured against the staged kernel on the vector units, FP16, 61
-// tilts: 512 x 128 x 256 voxels (512 workgroups), slabs of 46, 64 and 102
-// pixels: 1.10, 1.12 and 1.33 times as fast; 640 x 150 x 200 (800), 53: 0.87;
-// 256 x 64 x 256 (128), 64: 0.72; 768 x 100 x 100 (336), 150: 0.77. Lines of
-// whole 16-byte words, as others cost it the rest (483 x 156 x 400, 161: the
-// request 0.99). Of the volume's rows, not of a band's: the kernels differ in
-// the last bit.
+// With one slab always (61 tilts, 16 to 1000 pixels, 1 to 256 rows: nowhere
+// slower). With several, a workgroup's batches wait for window entries and
+// second runs in turn, which takes other workgroups to hide, wide slabs to be
+// rare, and full workgroups of 128 rows to pay. Its backprojection against the
+// staged kernel's, 41 tilts, slabs of 64 to 300 pixels:
+// - two workgroups per CU (512): 256 x 256 x 64 voxels (128) 0.79 to 1.04,
+//   512 rows of it (256) 0.98 to 1.29, 1024 (512) 1.22 to 1.60; 512 x 128 x 128
+//   (256) 0.90 to 1.24, 512 x 128 x 256 (512) 1.12 to 1.38;
+// - 32-row blocks that cost the staged kernel, 4 for about the time of 3.5, or
+//   of 2.75 where a last workgroup has 64 rows or less: of 512 x 256 and 1024 x
+//   256 tiles' worth, 32 rows 0.61 to 0.88, 96 0.89 to 1.18, 128 1.12 to 1.47,
+//   160 0.79 to 1.00, 192 0.92 to 1.18, 256 1.08 to 1.47, 320 0.98 to 1.27, 512
+//   1.12 to 1.36;
+// - slabs of at least 64 pixels (46: 1.10; 640 x 150 x 200, 53: 0.87);
+// - lines of whole 16-byte words, as others cost it the rest (483 x 156 x 400,
+//   161: the request 0.99).
+// Of the volume's rows, not of a band's: the kernels differ in the last bit.
 bool bp_mm_suits(int ndf, float dscale, int W, int Z, int Y) {
   if (ndf == 1) return true;
-  const size_t groups = (size_t)((W + kTile - 1) / kTile) *
-                        ((Z + kTile - 1) / kTile) * ((Y + 127) / 128);
-  return groups >= 512 && W % 4 == 0 && fabsf(dscale) * 64.0f <= 1.0f;
+  const int rest = Y % 128;
+  const size_t full = (size_t)Y / 128 + (rest > 64 ? 1 : 0);
+  const size_t half = rest > 0 && rest <= 64 ? 1 : 0;
+  const size_t tiles = (size_t)((W + kTile - 1) / kTile) *
+                       ((Z + kTile - 1) / kTile);
+  return tiles * (full + half) >= 512 &&
+         4 * ((size_t)(Y + 31) / 32) >= 14 * full + 11 * half && W % 4 == 0 &&
+         fabsf(dscale) * 64.0f <= 1.0f;
 }
 
 hipError_t launch_bp_mm(const BpArgs &a, int YB, int store, hipStream_t s) {

@@ -3,7 +3,8 @@ workgroup, one slab and several, each with a last workgroup of every number of
 row blocks, and values that are not finite in each.
 
 The forms are chosen by size: with one slab, more than 256 tiles of 16 x 16
-voxels times row groups take 128 or 64 rows; several slabs need 512.
+voxels times row groups take 128 or 64 rows; several slabs need 512, and rows
+that fill groups of 128 (so that 64 and 32 rows are left to calls for a band).
 """
 import numpy
 import pytest
@@ -21,7 +22,7 @@ ANGLES = numpy.deg2rad(numpy.linspace(-60, 60, T)).astype(f32)
 # X, Y, ndf, Z, W, (min_df, max_df)
 ONE = [(300, Y, 1, 256, 272, (0.0, 0.0))
        for Y in (32, 33, 64, 129, 161, 193, 225)]
-MULTI = [(520, Y, 3, 256, 512, (-130.0, 130.0)) for Y in (32, 40, 97, 161)]
+MULTI = [(520, Y, 3, 256, 512, (-130.0, 130.0)) for Y in (97, 225, 320, 321)]
 
 
 def run_plan(shape, storage, rows, sino, weights=None):
@@ -71,10 +72,36 @@ def test_row_groups(capi, shape, storage, rows):
 @pytest.mark.parametrize("shape", [
     (60, 2, 1, 496, 1540, (0.0, 0.0)), (60, 2, 1, 513, 1520, (0.0, 0.0)),
     (60, 2, 1, 512, 1521, (0.0, 0.0)), (60, 2, 1, 521, 1540, (0.0, 0.0)),
-    (60, 129, 1, 600, 1540, (0.0, 0.0)), (700, 2, 3, 513, 1536, (-300., 300.)),
+    (60, 129, 1, 600, 1540, (0.0, 0.0)), (700, 97, 3, 513, 1536, (-300., 300.)),
 ])
 def test_tile_orders(capi, shape):
     test_row_groups(capi, shape, "f16", 32)
+
+
+@pytest.mark.parametrize("storage", ["f16", "bf16"])
+@pytest.mark.parametrize("nan", [False, True])
+@pytest.mark.parametrize("shape", [ONE[6], MULTI[1]])
+def test_bands_of_rows_keep_the_bits(capi, shape, nan, storage):
+    # 32, 64 and 128 rows per workgroup, and a last row by itself
+    X, Y, ndf, Z, W, (mn, mx) = shape
+    sino = sinograms(shape)
+    if nan:
+        sino[[3, 70, 140], 0, 1, X // 2] = numpy.nan
+    plan = C.VolumePlan(X, Y, ANGLES, Z, width=W, num_defocus=ndf,
+                        centre=X / 2.0 - 0.3, min_defocus=mn, max_defocus=mx,
+                        storage=storage, input_layout=C.INPUT_SINOGRAMS)
+    assert plan.matrix_cores()
+    d_in = C.DeviceArray.from_host(sino)
+    d_vol = C.DeviceArray((Y, Z, W))
+    plan.run(d_in, d_vol)
+    C.call("gx_device_synchronize")
+    whole = d_vol.to_host()
+    for y0, y1 in ((0, 32), (32, 96), (96, 224), (224, Y)):
+        d_band = C.DeviceArray((y1 - y0, Z, W))
+        plan.backproject_rows(y0, y1, d_band)
+        C.call("gx_device_synchronize")
+        numpy.testing.assert_array_equal(d_band.to_host(), whole[y0:y1])
+    plan.destroy()
 
 
 @pytest.mark.parametrize("storage,rows", [("f16", 16), ("bf16", 32)])

@@ -52,7 +52,7 @@ def both(taps, weight, Z, W, angles, centre, mn, mx):
     (256, 3, 5, 1, 64, 256, (0.0, 0.0)),
     (256, 3, 16, 1, 64, 256, (0.0, 0.0)),
     (256, 2, 61, 1, 64, 256, (0.0, 0.0)),
-    (520, 130, 6, 3, 256, 512, (-130.0, 130.0)),
+    (520, 97, 6, 3, 256, 512, (-130.0, 130.0)),
 ])
 def test_no_further_off_than_fp32(capi, case, storage):
     X, Y, T, ndf, Z, W, (mn, mx) = case

@@ -14,11 +14,11 @@ from test_bp_mm_gpu import backproject, decoded
 
 pytestmark = pytest.mark.gpu
 
-# X, Y, T, ndf, Z, W, (min_df, max_df): one slab; three wide ones over 1024
-# workgroups, the last of each column with two rows
+# X, Y, T, ndf, Z, W, (min_df, max_df): one slab; three wide ones over 512
+# workgroups
 SHAPES = [
     (64, 40, 16, 1, 32, 64, (0.0, 0.0)),
-    (520, 130, 6, 3, 256, 512, (-130.0, 130.0)),
+    (520, 97, 6, 3, 256, 512, (-130.0, 130.0)),
 ]
 
 

@@ -12,7 +12,7 @@ def plan_of(width):
     """Three slabs `width` pixels wide; 512 workgroups."""
     angles = numpy.deg2rad(numpy.linspace(-60, 60, 5)).astype(numpy.float32)
     half = 1.5 * width
-    return C.VolumePlan(520, 40, angles, 256, width=512, num_defocus=3,
+    return C.VolumePlan(520, 97, angles, 256, width=512, num_defocus=3,
                         min_defocus=-half, max_defocus=half, storage="f16",
                         input_layout=C.INPUT_SINOGRAMS)
 
@@ -24,8 +24,8 @@ def lines(path):
 
 def test_kernels_have_their_own_choices(capi, tmp_path):
     C.tune_clear()
-    d_in = C.DeviceArray.from_host(numpy.ones((40, 3, 5, 520), numpy.float32))
-    d_vol = C.DeviceArray((40, 256, 512))
+    d_in = C.DeviceArray.from_host(numpy.ones((97, 3, 5, 520), numpy.float32))
+    d_vol = C.DeviceArray((97, 256, 512))
     # 100 pixels: the matrix cores; 40: the staged kernel, two slabs either way
     wide, narrow = plan_of(100), plan_of(40)
     assert wide.backprojector() == narrow.backprojector() == (C.BP_STAGED, 2)
@@ -50,3 +50,16 @@ def test_kernels_have_their_own_choices(capi, tmp_path):
     for q in (p, wide, narrow):
         q.destroy()
     C.tune_clear()
+
+
+@pytest.mark.parametrize("rows,matrix", [
+    (32, False), (96, False), (97, True), (128, True), (129, False),
+    (192, False), (193, True), (288, False), (320, True), (928, True),
+])
+def test_several_slabs_need_full_row_groups(capi, rows, matrix):
+    angles = numpy.zeros(1, numpy.float32)
+    p = C.VolumePlan(64, rows, angles, 256, width=512, num_defocus=2,
+                     min_defocus=-100.0, max_defocus=100.0, storage="f16",
+                     input_layout=C.INPUT_SINOGRAMS)
+    assert p.matrix_cores() == matrix
+    p.destroy()
